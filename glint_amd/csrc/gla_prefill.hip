@@ -17,6 +17,8 @@
 // register shuffle between the two products.
 #include <math.h>
 
+#include <algorithm>
+
 #include "gla_internal.h"
 
 namespace gla {
@@ -70,11 +72,44 @@ __device__ __forceinline__ float sum_rows4(float x) {
     return __uint_as_float(c[0]) + __uint_as_float(c[1]);
 }
 
-__device__ __forceinline__ float tanh_approx(float x) {
-    float t = fast_exp2(-2.0f * kLog2e * fabsf(x));
-    float r = (1.0f - t) / (1.0f + t);
-    return copysignf(r, x);
+// max / min of unsigned words over the wave, in every lane: DPP rotations within
+// each 16-lane row, then the row swaps.
+template <bool MAX>
+__device__ __forceinline__ uint32_t wave_extreme(uint32_t x) {
+    const auto pick = [](uint32_t a, uint32_t b) { return MAX ? max(a, b) : min(a, b); };
+    x = pick(x, __builtin_amdgcn_update_dpp(0, x, 0x121, 0xf, 0xf, true));  // row_ror 1, 2, 4, 8
+    x = pick(x, __builtin_amdgcn_update_dpp(0, x, 0x122, 0xf, 0xf, true));
+    x = pick(x, __builtin_amdgcn_update_dpp(0, x, 0x124, 0xf, 0xf, true));
+    x = pick(x, __builtin_amdgcn_update_dpp(0, x, 0x128, 0xf, 0xf, true));
+    const auto a = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    x = pick(a[0], a[1]);
+    const auto c = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return pick(c[0], c[1]);
 }
+__device__ __forceinline__ uint32_t umax_rows4(uint32_t x) {
+    const auto a = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    x = max(a[0], a[1]);
+    const auto c = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return max(c[0], c[1]);
+}
+
+// cap * tanh(x / cap) * log2(e), without the long division sequences: x / cap
+// by the reciprocal of cap and one correction, 1 / (1 + t) by v_rcp_f32 and one
+// Newton step (each then within an ulp).
+struct SoftCap {
+    float cap, inv, out;
+    __device__ __forceinline__ explicit SoftCap(float c) : cap(c), inv(1.0f / c), out(c * kLog2e) {}
+    __device__ __forceinline__ float operator()(float x) const {
+        const float q = x * inv;
+        // past 16 tanh is 1, and an infinite score has no remainder
+        const float y = fabsf(q) < 16.0f ? fmaf(fmaf(-cap, q, x), inv, q) : q;
+        const float t = fast_exp2(-2.0f * kLog2e * fabsf(y));
+        const float d = 1.0f + t;
+        float r = __builtin_amdgcn_rcpf(d);
+        r = fmaf(fmaf(-d, r, 1.0f), r, r);
+        return copysignf((1.0f - t) * r * out, x);
+    }
+};
 
 // Soft-cap and causal/window mask of one query column of a 32-key score tile
 // (sacc[mt][i]: key k0 + 16*mt + 4*lgrp + i), in place, log2 domain. The
@@ -85,10 +120,11 @@ template <bool CAP>
 __device__ __forceinline__ void cap_and_mask(floatx4 (&s)[2], float softcap, bool interior, int kbase, int qpos,
                                              int qlo, int klo, int khi) {
     if constexpr (CAP) {
+        const SoftCap f(softcap);
 #pragma unroll
         for (int mt = 0; mt < 2; mt++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) s[mt][i] = softcap * tanh_approx(s[mt][i] / softcap) * kLog2e;
+            for (int i = 0; i < 4; i++) s[mt][i] = f(s[mt][i]);
     }
     if (!interior) {
         const int lo = max(qlo, klo), hi = min(qpos, khi);
@@ -219,32 +255,29 @@ __device__ __forceinline__ void store_tile(const TileRegs<D, NTHR> &t, float *Ks
 // O^T row R of d-tile t is d = R*DT + t, so the V^T operands a lane needs
 // for one key are DT consecutive floats, and a lane's outputs for a query
 // are the 4*DT consecutive floats [4g*DT, 4(g+1)*DT).
+template <int D>
+constexpr int kF32Lds = 4 * KT * kRow<D> * 4;  // two K and two V tiles
+
 template <int D, int NT, int NW, bool Q8, bool CAP>
-__global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(const PrefillParams p) {
+__device__ __forceinline__ void prefill_f32_body(const PrefillParams &p, uint8_t *lds, int unit, int qb0) {
     constexpr int NTHR = NW * 64;
     constexpr int QW = 16 * NT;  // queries per wave
     constexpr int KS = D / 4;    // k-steps of S = K Q^T
     constexpr int DT = D / 16;   // d tiles of O
-    __shared__ __attribute__((aligned(16))) float Ks[2][KT * kRow<D>];
-    __shared__ __attribute__((aligned(16))) float Vs[2][KT * kRow<D>];
+    float *Kb = reinterpret_cast<float *>(lds);
+    float *Vb = Kb + 2 * KT * kRow<D>;
 
-    // grid (sequence x KV head x head group, query block): every unit's
-    // longest (last) query block is dispatched before any shorter one, so the
-    // grid ends on short workgroups
     const int n_hgrp = p.group / p.hpw;
-    const int unit = blockIdx.x;
     const int b = unit / (p.n_kv_heads * n_hgrp);
     const int kvh = (unit - b * p.n_kv_heads * n_hgrp) / n_hgrp;
     const int hgrp = unit - (b * p.n_kv_heads + kvh) * n_hgrp;
-    const int qblk = p.n_qblocks - 1 - (int)blockIdx.y;
     const int waves_per_head = NW / p.hpw;
     const int qwg = QW * waves_per_head;
 
     const int row0 = p.q_start[b];
     const int q_len = min(max(p.q_start[b + 1] - row0, 0), p.max_q_len);
     const int pos0 = p.pos_offset[b];
-    const int qb0 = qblk * qwg;  // first local query of the workgroup
-    if (qb0 >= q_len) return;
+    if (qb0 >= q_len) return;  // qb0: first local query
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -297,14 +330,14 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(const PrefillParam
         const int kfirst = (klo / KT) * KT;
         TileRegs<D, NTHR> tr;
         fetch_tile<D, NTHR, Q8>(p, b, kvh, kfirst, klo, khi, tr);
-        store_tile<D, NTHR, Q8>(tr, Ks[0], Vs[0]);
+        store_tile<D, NTHR, Q8>(tr, Kb, Vb);
         __syncthreads();
         int buf = 0;
         for (int k0 = kfirst; k0 <= khi; k0 += KT, buf ^= 1) {
             const bool more = k0 + KT <= khi;
             if (more) fetch_tile<D, NTHR, Q8>(p, b, kvh, k0 + KT, klo, khi, tr);
-            const float *ks = Ks[buf];
-            const float *vs = Vs[buf];
+            const float *ks = Kb + buf * KT * kRow<D>;
+            const float *vs = Vb + buf * KT * kRow<D>;
 
             // S^T = K . Q^T
             floatx4 sacc[2][NT];
@@ -400,7 +433,7 @@ __global__ __launch_bounds__(NW * 64) void prefill_f32_kernel(const PrefillParam
                 }
             }
 
-            if (more) store_tile<D, NTHR, Q8>(tr, Ks[buf ^ 1], Vs[buf ^ 1]);
+            if (more) store_tile<D, NTHR, Q8>(tr, Kb + (buf ^ 1) * KT * kRow<D>, Vb + (buf ^ 1) * KT * kRow<D>);
             __syncthreads();
         }
     }
@@ -1247,6 +1280,599 @@ __global__ __launch_bounds__(kBf16sWaves<D> * 64, kBf16sOccupancy<D>) void prefi
     }
 }
 
+// ---------------------------------------------------------------------------
+// fp32 prefill on the f16 matrix cores. Every f32 operand is two f16 pieces
+// (hi = f16(x), lo = f16(x - hi): 22 bits) after a power-of-two scaling, and a
+// product is three MFMAs, hi.hi + hi.lo + lo.hi; the dropped lo.lo is 2^-24 of
+// the product. Products of f16 pieces are exact in the f32 accumulators, and a
+// 32-wide MFMA rounds once where the 4-wide f32 one rounds eight times, so the
+// error against 64 bits does not grow: 4 prompts of 2,048 at 32/8 heads, d =
+// 128, have a relative error of 2.7e-7 (f32 MFMAs: 4.4e-7). Three f16 MFMAs do
+// the work of a 16x16x32 tile in 48 cycles, the f32 ones in 256: the same four
+// prompts take 375 us, of them 23 the staging (f32 MFMAs: 1,083 us), 367
+// TFLOP/s. What bounds it is the chain S -> softmax -> O at two waves per SIMD:
+// a tile takes a workgroup 2.2 us and its MFMAs 0.65 us of each wave's SIMD.
+//
+// Scaling. K takes one power of two per 32-key tile, undone on the scores (with
+// the query's own); V one per tile as well, which is the unit O is accumulated
+// in: when it changes, O is moved to the new unit (an exact product). The
+// exponents are rounded up to multiples of 4, so tiles of like magnitude share
+// a unit. p = 2^(s - m) is held below 2^14 (kSplitP).
+//
+// What the pieces cannot carry at f32 precision goes through the f32 body
+// above, decided per workgroup: a tile that holds an infinity or a NaN, whose
+// largest value lies outside [2^-45, 2^45] (K) or [2^-20, 2^20] (V), or whose
+// values differ too much in magnitude (kSplitRange), and a query row with a
+// non-finite value or a maximum outside [2^-45, 2^45]. A value x of a tile whose
+// largest is M has an error of at most max(2^-23 |x|, 2^-35 M).
+typedef _Float16 half8p __attribute__((ext_vector_type(8)));
+
+constexpr int kSplitP = 6;            // p is scaled by 2^6: with the lazy maximum's 2^8 it stays below 2^14
+// How much smaller than a tile's largest value that of 8 dims of a key (K) or
+// of 8 keys of a dim (V) may be: 2^12; in a tile that is not full 2^20, since
+// there a V run may hold one key, whose value is small by chance.
+constexpr float kSplitRange = 0x1p12f, kSplitRangePart = 0x1p20f;
+
+// A tile's image: K hi, K lo, V hi, V lo, each 64*D bytes in the piece order
+// of the bf16 image.
+template <int D>
+constexpr int kSplitImage = 256 * D;
+// What the attention needs to know of a tile: the factor that undoes K's
+// scale (NaN: the tile takes the f32 body), and V's scale (0: V is all zero).
+struct TileMeta {
+    float k_inv, v_scale;
+};
+
+__device__ __forceinline__ void split8(const float (&x)[8], float mul, half8p &hi, half8p &lo) {
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const float t = x[j] * mul;
+        const _Float16 h = (_Float16)t;
+        hi[j] = h;
+        lo[j] = (_Float16)(t - (float)h);
+    }
+}
+
+// 2^(14 - e) for the exponent e of m (m in [2^(e-1), 2^e)), e rounded up to a
+// multiple of STEP: m times it lies in [2^(14-STEP), 2^14).
+template <int STEP>
+__device__ __forceinline__ int split_exponent(float m) {
+    int e = (int)((__float_as_uint(m) >> 23) & 0xff) - 126;
+    e = (e + STEP - 1) & ~(STEP - 1);
+    return 14 - e;
+}
+__device__ __forceinline__ float pow2f(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
+
+// One 32-key tile of a (sequence, KV head) pair on its way from the cache to
+// its pieces, by 256 threads: fetch() issues the loads, convert() finds the
+// tile's scales and hands out the pieces.
+// K piece i is 8 consecutive dims of one key, V piece i 8 keys of one dim.
+template <int D>
+__device__ __forceinline__ int k_piece_key(int i) { return i / (D / 8 * 16) * 16 + (i & 15); }
+template <int D>
+__device__ __forceinline__ int k_piece_dim(int i) { return (i % (D / 8 * 16) >> 4) * 8; }
+__device__ __forceinline__ int v_piece_key(int i, int j) { return (j >> 2) * 16 + 4 * ((i >> 4) & 3) + (j & 3); }
+__device__ __forceinline__ int v_piece_dim(int i) { return 16 * (i >> 6) + (i & 15); }
+
+// What convert() needs in LDS.
+template <int D, bool Q8>
+struct SplitAux {
+    uint4 ext[4];  // per wave, as bits: largest |K|, smallest non-zero run maximum of K; the same of V
+    TileMeta meta;
+    uint32_t pad[2];
+    float v[Q8 ? 1 : KT][Q8 ? 4 : D + 4];  // f32 rows of V, read back along the keys
+};
+
+template <int D, bool Q8>
+struct SplitTile {
+    static constexpr int NK = 4 * D / 256;  // 16-byte pieces of K (and of V) per thread
+    // f32: the rows' own 16-byte loads; Q8_0: quants and scales
+    floatx4 ka[Q8 ? 1 : NK][2], va[Q8 ? 1 : NK][2];
+    uint2 kw[Q8 ? NK : 1];
+    uint32_t vw[Q8 ? NK : 1][2];
+    uint16_t ks[Q8 ? NK : 1], vs[Q8 ? NK : 1][8];
+
+    // keys outside [klo, khi] are zero (khi >= 0, and the tile meets the range)
+    __device__ __forceinline__ void fetch(const PrefillParams &p, int b, int kvh, int k0, int klo, int khi) {
+        const int64_t head_off = (int64_t)kvh * p.kv.head_stride;
+        const int64_t hb0 = map_page(p.pm, b, min(k0, khi) >> 4) * p.kv.page_stride + head_off;
+        const int64_t hb1 = map_page(p.pm, b, min(k0 + 16, khi) >> 4) * p.kv.page_stride + head_off;
+        if constexpr (Q8) {
+#pragma unroll
+            for (int r = 0; r < NK; r++) {
+                const int i = threadIdx.x + 256 * r;
+                const int key = k_piece_key<D>(i), d = k_piece_dim<D>(i);
+                const int64_t hb = key < 16 ? hb0 : hb1;
+                kw[r] = *reinterpret_cast<const uint2 *>(p.kv.k + hb + q8k_off(key & 15, d, D));
+                ks[r] = reinterpret_cast<const uint16_t *>(p.kv.ks + hb)[q8ks_off(key & 15, d >> 5, D)];
+                const int vd = v_piece_dim(i), g4 = 4 * ((i >> 4) & 3);
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const int64_t vb = h ? hb1 : hb0;
+                    vw[r][h] = *reinterpret_cast<const uint32_t *>(p.kv.v + vb + q8v_off(g4, vd, D));
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        vs[r][4 * h + j] =
+                            reinterpret_cast<const uint16_t *>(p.kv.vs + vb)[(g4 + j) * (D / 32) + (vd >> 5)];
+                }
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < NK; r++) {
+                const int u = threadIdx.x + 256 * r;
+                const int key = u / (D / 8);
+                const int kp = k0 + key;
+                va[r][0] = va[r][1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                if (kp >= klo && kp <= khi) {
+                    const float *vr = reinterpret_cast<const float *>(p.kv.v + (key < 16 ? hb0 : hb1) +
+                                                                      (int64_t)(kp & 15) * p.kv.row_stride) +
+                                      8 * (u - key * (D / 8));
+                    va[r][0] = *reinterpret_cast<const floatx4 *>(vr);
+                    va[r][1] = *reinterpret_cast<const floatx4 *>(vr + 4);
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < NK; r++) {
+                const int i = threadIdx.x + 256 * r;
+                const int key = k_piece_key<D>(i);
+                const int kp = k0 + key;
+                ka[r][0] = ka[r][1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                if (kp >= klo && kp <= khi) {
+                    const float *kr = reinterpret_cast<const float *>(p.kv.k + (key < 16 ? hb0 : hb1) +
+                                                                      (int64_t)(kp & 15) * p.kv.row_stride) +
+                                      k_piece_dim<D>(i);
+                    ka[r][0] = *reinterpret_cast<const floatx4 *>(kr);
+                    ka[r][1] = *reinterpret_cast<const floatx4 *>(kr + 4);
+                }
+            }
+        }
+    }
+
+    // put(i, k_hi, k_lo, v_hi, v_lo) takes piece i of each image, unless the
+    // pieces cannot carry the tile (aux.meta.k_inv is NaN). No thread may
+    // still be reading aux; after the next barrier aux.meta may be read.
+    template <typename Put>
+    __device__ __forceinline__ void convert(SplitAux<D, Q8> &aux, int k0, int klo, int khi, Put put) const {
+        float kf[NK][8], vf[NK][8];
+        if constexpr (!Q8) {
+#pragma unroll
+            for (int r = 0; r < NK; r++) {
+                const int u = threadIdx.x + 256 * r;
+                const int key = u / (D / 8);
+                floatx4 *dst = reinterpret_cast<floatx4 *>(&aux.v[key][8 * (u - key * (D / 8))]);
+                dst[0] = va[r][0];
+                dst[1] = va[r][1];
+            }
+            __syncthreads();
+        }
+#pragma unroll
+        for (int r = 0; r < NK; r++) {
+            const int i = threadIdx.x + 256 * r;
+            if constexpr (Q8) {
+                const int kp = k0 + k_piece_key<D>(i);
+                const bool ok = kp >= klo && kp <= khi;
+                const float ksc = __half2float(__ushort_as_half(ks[r]));
+#pragma unroll
+                for (int j = 0; j < 8; j++) {  // stored quants are x + 128
+                    const uint32_t w = j < 4 ? kw[r].x : kw[r].y;
+                    kf[r][j] = ok ? (float)((int)((w >> (8 * (j & 3))) & 0xff) - 128) * ksc : 0.0f;
+                    const int vp = k0 + v_piece_key(i, j);
+                    const float vsc = __half2float(__ushort_as_half(vs[r][j]));
+                    vf[r][j] = vp >= klo && vp <= khi
+                                   ? (float)((int)((vw[r][j >> 2] >> (8 * (j & 3))) & 0xff) - 128) * vsc
+                                   : 0.0f;
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    kf[r][j] = ka[r][j >> 2][j & 3];
+                    vf[r][j] = aux.v[v_piece_key(i, j)][v_piece_dim(i)];
+                }
+            }
+        }
+        // magnitudes, as the bits of |x| (an infinity or a NaN is the largest)
+        uint32_t ktop = 0, klow = 0xffffffffu, vtop = 0, vlow = 0xffffffffu;
+#pragma unroll
+        for (int r = 0; r < NK; r++) {
+            uint32_t km = 0, vm = 0;
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                km = max(km, __float_as_uint(kf[r][j]) & 0x7fffffffu);
+                vm = max(vm, __float_as_uint(vf[r][j]) & 0x7fffffffu);
+            }
+            ktop = max(ktop, km);
+            klow = min(klow, km ? km : 0xffffffffu);
+            vtop = max(vtop, vm);
+            vlow = min(vlow, vm ? vm : 0xffffffffu);
+        }
+        const uint4 mine = make_uint4(wave_extreme<true>(ktop), wave_extreme<false>(klow), wave_extreme<true>(vtop),
+                                      wave_extreme<false>(vlow));
+        if ((threadIdx.x & 63) == 0) aux.ext[threadIdx.x >> 6] = mine;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const uint4 x = aux.ext[w];
+            ktop = max(w ? ktop : 0, x.x);
+            klow = min(w ? klow : 0xffffffffu, x.y);
+            vtop = max(w ? vtop : 0, x.z);
+            vlow = min(w ? vlow : 0xffffffffu, x.w);
+        }
+        const float kmax = __uint_as_float(ktop), vmax = __uint_as_float(vtop);
+        const float range = k0 >= klo && k0 + KT - 1 <= khi ? kSplitRange : kSplitRangePart;
+        bool plain = ktop < 0x7f800000u && vtop < 0x7f800000u;
+        int ke = 0, ve = 0;
+        if (plain && ktop) {
+            plain = kmax >= 0x1p-45f && kmax <= 0x1p45f && __uint_as_float(klow) * range >= kmax;
+            ke = split_exponent<4>(kmax);
+        }
+        if (plain && vtop) {
+            plain = vmax >= 0x1p-20f && vmax <= 0x1p20f && __uint_as_float(vlow) * range >= vmax;
+            ve = split_exponent<4>(vmax);
+        }
+        if (threadIdx.x == 0)
+            aux.meta = TileMeta{plain ? pow2f(-ke) : __uint_as_float(0x7fc00000u), vtop ? pow2f(ve) : 0.0f};
+        if (!plain) return;
+        const float kmul = pow2f(ke), vmul = pow2f(ve);
+#pragma unroll
+        for (int r = 0; r < NK; r++) {
+            half8p kh, kl, vh, vl;
+            split8(kf[r], kmul, kh, kl);
+            split8(vf[r], vmul, vh, vl);
+            put(threadIdx.x + 256 * r, kh, kl, vh, vl);
+        }
+    }
+};
+
+// Grid (tile, (sequence, KV head) pair), 256 threads.
+template <int D, bool Q8>
+__global__ __launch_bounds__(256) void stage_split_kernel(const PrefillParams p, uint8_t *img, TileMeta *meta,
+                                                          int n_tiles, int pair0) {
+    const int t = blockIdx.x;
+    const int pair = pair0 + blockIdx.y;
+    const int b = pair / p.n_kv_heads;
+    const int kvh = pair - b * p.n_kv_heads;
+    const int row0 = p.q_start[b];
+    const int q_len = min(max(p.q_start[b + 1] - row0, 0), p.max_q_len);
+    if (q_len == 0) return;
+    const int pos0 = p.pos_offset[b];
+    const int khi = min(pos0 + q_len - 1, p.pm.pos_limit - 1);
+    const int klo = window_lo(pos0, p.sliding_window);
+    const int k0 = t * KT;
+    if (khi < klo || k0 > khi || k0 + KT - 1 < klo) return;  // a tile no query of the sequence reads
+
+    __shared__ __attribute__((aligned(16))) SplitAux<D, Q8> aux;
+    SplitTile<D, Q8> tile;
+    tile.fetch(p, b, kvh, k0, klo, khi);
+    const int64_t at = (int64_t)blockIdx.y * n_tiles + t;
+    uint8_t *dst = img + at * kSplitImage<D>;
+    tile.convert(aux, k0, klo, khi, [&](int i, const half8p &kh, const half8p &kl, const half8p &vh, const half8p &vl) {
+        *reinterpret_cast<half8p *>(dst + (int64_t)i * 16) = kh;
+        *reinterpret_cast<half8p *>(dst + 64 * D + (int64_t)i * 16) = kl;
+        *reinterpret_cast<half8p *>(dst + 128 * D + (int64_t)i * 16) = vh;
+        *reinterpret_cast<half8p *>(dst + 192 * D + (int64_t)i * 16) = vl;
+    });
+    if (threadIdx.x == 0) meta[at] = aux.meta;
+}
+
+// Waves per SIMD the kernel's registers are sized for; LDS holds two tiles of
+// a workgroup (or the f32 body's buffers): d = 64 35 KB, d = 128 68 KB,
+// d = 256 133 KB. A workgroup that converts its own tiles holds one image and
+// the conversion's buffers, and the next tile's loads in registers (not at
+// d = 256, whose registers are full).
+template <int D, bool STAGED>
+constexpr int kSplitOccupancy = !STAGED ? (D == 64 ? 2 : 1) : (D == 64 ? 3 : (D == 128 ? 2 : 1));
+// 16-query tiles per wave: two share every operand read; the few rows of an
+// unstaged call are spread over more waves instead.
+template <bool STAGED>
+constexpr int kSplitNT = STAGED ? 2 : 1;
+
+template <int D, bool Q8, bool CAP, bool STAGED>
+__global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED>)) void prefill_split_kernel(const PrefillParams p,
+                                                                                const uint8_t *img,
+                                                                                const TileMeta *meta, int n_tiles,
+                                                                                int pair0) {
+    constexpr int NW = 4, NT = kSplitNT<STAGED>;
+    constexpr int QW = 16 * NT;
+    constexpr int KS = D / 32;
+    constexpr int DT = D / 16;
+    constexpr int IMG = kSplitImage<D>;
+    constexpr int CPW = IMG / 1024 / NW;  // kilobyte copies per wave and tile
+    constexpr int AUX = IMG + (int)sizeof(SplitAux<D, Q8>);
+    constexpr int LDS = std::max(kF32Lds<D>, STAGED ? 2 * IMG : AUX);
+    __shared__ __attribute__((aligned(16))) uint8_t lds[LDS];
+
+    const int n_hgrp = p.group / p.hpw;
+    const int unit = pair0 * n_hgrp + (int)blockIdx.x;
+    const int pair = unit / n_hgrp;
+    const int b = pair / p.n_kv_heads;
+    const int kvh = pair - b * p.n_kv_heads;
+    const int hgrp = unit - pair * n_hgrp;
+    const int qblk = p.n_qblocks - 1 - (int)blockIdx.y;
+    const int waves_per_head = NW / p.hpw;
+    const int qwg = QW * waves_per_head;
+
+    const int row0 = p.q_start[b];
+    const int q_len = min(max(p.q_start[b + 1] - row0, 0), p.max_q_len);
+    const int pos0 = p.pos_offset[b];
+    const int qb0 = qblk * qwg;
+    if (qb0 >= q_len) return;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lrow = lane & 15;
+    const int lgrp = lane >> 4;
+    const int head = kvh * p.group + hgrp * p.hpw + (wave % p.hpw);
+    const int wq0 = qb0 + (wave / p.hpw) * QW;
+
+    const int q_last = min(q_len, qb0 + qwg) - 1;
+    const int khi = min(pos0 + q_last, p.pm.pos_limit - 1);
+    const int klo = window_lo(pos0 + qb0, p.sliding_window);
+    const int tfirst = klo / KT;
+    const int n = khi >= klo ? khi / KT - tfirst + 1 : 0;
+    const TileMeta *unit_meta = meta + (int64_t)(pair - pair0) * n_tiles + tfirst;
+    const uint8_t *unit_img = img + ((int64_t)(pair - pair0) * n_tiles + tfirst) * IMG;
+    const uint32_t ring = __builtin_amdgcn_readfirstlane(
+        (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)&lds[0]);
+    auto issue = [&](int i) {
+        const uint8_t *src = unit_img + (int64_t)i * IMG;
+        const uint32_t dst = ring + (uint32_t)((i & 1) * IMG);
+#pragma unroll
+        for (int c = 0; c < CPW; c++) {
+            const int piece = wave * CPW + c;
+            lds_copy16(src, (uint32_t)(piece * 1024 + lane * 16), dst + piece * 1024);
+        }
+    };
+
+    if (STAGED && n > 0) issue(0);
+    // tiles and queries that the pieces cannot carry
+    bool odd = false;
+    for (int i = tid; STAGED && i < n; i += 256) odd = odd || unit_meta[i].k_inv != unit_meta[i].k_inv;
+
+    // Q^T operand: pieces of Q[query nt*16 + lrow][d = ks*32 + lgrp*8 + 0..7]
+    // times the query's own power of two
+    half8p qh[NT][KS], ql[NT][KS];
+    float qinv[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) {
+        const int lq = wq0 + nt * 16 + lrow;
+        const bool ok = lq < q_len;
+        const float *qp = p.q + ((int64_t)(row0 + (ok ? lq : 0)) * p.n_heads + head) * D;
+        float x[KS][8];
+        uint32_t mx = 0;
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            const floatx4 a = __builtin_nontemporal_load(reinterpret_cast<const floatx4 *>(qp + ks * 32 + lgrp * 8));
+            const floatx4 c = __builtin_nontemporal_load(reinterpret_cast<const floatx4 *>(qp + ks * 32 + lgrp * 8 + 4));
+#pragma unroll
+            for (int j = 0; j < 8; j++) x[ks][j] = ok ? (j < 4 ? a[j & 3] : c[j & 3]) * p.q_mul : 0.0f;
+        }
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+            for (int j = 0; j < 8; j++) mx = max(mx, __float_as_uint(x[ks][j]) & 0x7fffffffu);
+        mx = umax_rows4(mx);
+        const float top = __uint_as_float(mx);
+        const bool fits = mx == 0 || (top >= 0x1p-45f && top <= 0x1p45f);  // false for an infinity or a NaN
+        odd = odd || !fits;
+        const int e = mx && fits ? split_exponent<1>(top) : 0;
+        qinv[nt] = pow2f(-e);
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) split8(x[ks], pow2f(e), qh[nt][ks], ql[nt][ks]);
+    }
+    if (STAGED) wait_vm<0>();  // the first tile has landed, so the f32 body may use its place
+    const auto in_f32 = [&]() {
+        constexpr int FT = D == 256 ? 1 : NT;  // d = 256: half a wave's queries at a time, more would spill
+        for (int q = qb0; q < qb0 + qwg; q += 16 * FT * waves_per_head) {
+            __syncthreads();  // the LDS is free
+            prefill_f32_body<D, FT, NW, Q8, CAP>(p, lds, unit, q);
+        }
+    };
+    bool f32 = __syncthreads_or(odd);
+    if (STAGED && f32) {
+        in_f32();
+        return;
+    }
+
+    floatx4 o[DT][NT];
+    float m[NT], lpart[NT];
+    int qpos[NT], qlo[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) {
+#pragma unroll
+        for (int t = 0; t < DT; t++) o[t][nt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        lpart[nt] = 0.0f;
+        m[nt] = kMInit;
+        const int lq = wq0 + nt * 16 + lrow;
+        qpos[nt] = lq < q_len ? pos0 + lq : -1;
+        qlo[nt] = window_lo(pos0 + lq, p.sliding_window);
+    }
+    // keys this wave's queries attend: [wlo, whi]
+    const int whi = min(khi, pos0 + wq0 + QW - 1);
+    const int wlo = max(klo, window_lo(pos0 + wq0, p.sliding_window));
+    float unit_v = 0.0f;  // O's unit: the scale of the last tile's V (0: none yet)
+
+    auto attend = [&](int i, const uint8_t *kimg, const TileMeta &cur) {
+        const int k0 = (tfirst + i) * KT;
+        if (k0 > whi || k0 + KT - 1 < wlo) return;  // no query of this wave attends it
+
+        // S^T = K . Q^T: the hi products and the cross terms apart, added at
+        // the end (the small terms are not rounded at the large ones' unit)
+        floatx4 s[2][NT], x[2][NT];
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                s[mt][nt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                x[mt][nt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            half8p ah[2], al[2];
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) {
+                const uint8_t *src = kimg + ((mt * (D / 8) + ks * 4 + lgrp) * 16 + lrow) * 16;
+                ah[mt] = *reinterpret_cast<const half8p *>(src);
+                al[mt] = *reinterpret_cast<const half8p *>(src + 64 * D);
+            }
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++)
+                    s[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[mt], qh[nt][ks], s[mt][nt], 0, 0, 0);
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++)
+                    x[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[mt], ql[nt][ks], x[mt][nt], 0, 0, 0);
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++)
+                    x[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[mt], qh[nt][ks], x[mt][nt], 0, 0, 0);
+        }
+
+        // softmax: as the bf16 kernels' (a lazy maximum), in f32; c undoes the scales
+        const bool interior = k0 >= klo && k0 + KT - 1 <= min(khi, pos0 + wq0) &&
+                              (p.sliding_window <= 0 || k0 >= window_lo(pos0 + wq0 + QW - 1, p.sliding_window));
+        half8p ph[NT], pl[NT];
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) {
+            float c = cur.k_inv * qinv[nt];
+            floatx4 col[2] = {s[0][nt] + x[0][nt], s[1][nt] + x[1][nt]};
+            if constexpr (CAP) {
+                col[0] *= c;
+                col[1] *= c;
+                c = 1.0f;
+            }
+            cap_and_mask<CAP>(col, p.softcap, interior, k0 + 4 * lgrp, qpos[nt], qlo[nt], klo, khi);
+            float mx = max3f(max3f(col[0][0], col[0][1], col[0][2]), max3f(col[0][3], col[1][0], col[1][1]),
+                             max2f(col[1][2], col[1][3])) * c;
+            if (__ballot(mx - m[nt] > kLazyMax)) {
+                mx = max_rows4(mx);
+                const bool up = mx - m[nt] > kLazyMax;
+                const float rs = up ? fast_exp2(m[nt] - mx) : 1.0f;
+                m[nt] = up ? mx : m[nt];
+#pragma unroll
+                for (int t = 0; t < DT; t++) o[t][nt] *= rs;
+                lpart[nt] *= rs;
+            }
+            const float sub = (float)kSplitP - m[nt];
+            float ls = 0.0f;
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float pv = fast_exp2(fmaf(col[mt][r], c, sub));
+                    ls += pv;
+                    const _Float16 h = (_Float16)pv;
+                    ph[nt][4 * mt + r] = h;
+                    pl[nt][4 * mt + r] = (_Float16)(pv - (float)h);
+                }
+            lpart[nt] += ls;
+        }
+
+        // O^T += V^T . P^T in V's unit
+        if (cur.v_scale == 0.0f) return;
+        if (cur.v_scale != unit_v) {
+            const float f = unit_v == 0.0f ? 1.0f : cur.v_scale / unit_v;
+#pragma unroll
+            for (int t = 0; t < DT; t++)
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++) o[t][nt] *= f;
+            unit_v = cur.v_scale;
+        }
+        const uint8_t *vimg = kimg + 128 * D;
+#pragma unroll
+        for (int t = 0; t < DT; t++) {
+            const uint8_t *src = vimg + ((t * 4 + lgrp) * 16 + lrow) * 16;
+            const half8p ah = *reinterpret_cast<const half8p *>(src);
+            const half8p al = *reinterpret_cast<const half8p *>(src + 64 * D);
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++)
+                o[t][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, ph[nt], o[t][nt], 0, 0, 0);
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++)
+                o[t][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, pl[nt], o[t][nt], 0, 0, 0);
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++)
+                o[t][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, ph[nt], o[t][nt], 0, 0, 0);
+        }
+    };
+
+    if constexpr (STAGED) {
+        TileMeta tm = n > 0 ? unit_meta[0] : TileMeta{1.0f, 0.0f};
+        for (int i = 0; i < n; i++) {
+            // this wave's copies of tile i have landed, then every wave's; every
+            // wave is also done with tile i - 1, whose buffer the next copy takes
+            wait_vm<0>();
+            __syncthreads();
+            if (i + 1 < n) issue(i + 1);
+            const TileMeta cur = tm;
+            tm = unit_meta[min(i + 1, n - 1)];
+            attend(i, lds + (i & 1) * IMG, cur);
+        }
+    } else if (n > 0 && !f32) {
+        SplitAux<D, Q8> &aux = *reinterpret_cast<SplitAux<D, Q8> *>(lds + IMG);
+        // the keys that a staged tile would hold: what any query of the sequence attends
+        const int ulo = window_lo(pos0, p.sliding_window);
+        const int uhi = min(pos0 + q_len - 1, p.pm.pos_limit - 1);
+        constexpr bool AHEAD = D < 256;
+        SplitTile<D, Q8> tile;
+        tile.fetch(p, b, kvh, tfirst * KT, ulo, uhi);
+        for (int i = 0; i < n; i++) {
+            const int k0 = (tfirst + i) * KT;
+            if (!AHEAD && i > 0) tile.fetch(p, b, kvh, k0, ulo, uhi);
+            tile.convert(aux, k0, ulo, uhi, [&](int j, const half8p &kh, const half8p &kl, const half8p &vh, const half8p &vl) {
+                *reinterpret_cast<half8p *>(lds + j * 16) = kh;
+                *reinterpret_cast<half8p *>(lds + 64 * D + j * 16) = kl;
+                *reinterpret_cast<half8p *>(lds + 128 * D + j * 16) = vh;
+                *reinterpret_cast<half8p *>(lds + 192 * D + j * 16) = vl;
+            });
+            __syncthreads();
+            const TileMeta cur = aux.meta;
+            if (cur.k_inv != cur.k_inv) {
+                f32 = true;
+                break;
+            }
+            if (AHEAD && i + 1 < n) tile.fetch(p, b, kvh, k0 + KT, ulo, uhi);
+            attend(i, lds, cur);
+            __syncthreads();  // before the next tile takes its place
+        }
+    }
+
+    if (!STAGED && f32) {
+        in_f32();
+        return;
+    }
+
+    // Output rows through LDS, as the staged bf16 kernel writes them
+    constexpr int SROW = D + 4;
+    static_assert(NW * 16 * SROW * 4 <= LDS, "output staging fits");
+    __syncthreads();
+    float *stage = reinterpret_cast<float *>(lds) + wave * 16 * SROW;
+    constexpr int LPR = D / 4;    // lanes per row (16 bytes each)
+    constexpr int RPI = 64 / LPR;  // rows per store instruction
+    const float unscale = unit_v == 0.0f ? 1.0f : 1.0f / unit_v;
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) {
+        const float lt = sum_rows4(lpart[nt]);
+        const float inv = lt > 0.0f ? 1.0f / lt * unscale : 0.0f;
+#pragma unroll
+        for (int t = 0; t < DT; t++)
+            *reinterpret_cast<floatx4 *>(stage + lrow * SROW + 16 * t + 4 * lgrp) = o[t][nt] * inv;
+#pragma unroll
+        for (int k = 0; k < 16 / RPI; k++) {
+            const int r = k * RPI + lane / LPR;
+            const int c = (lane % LPR) * 4;
+            const floatx4 v = *reinterpret_cast<const floatx4 *>(stage + r * SROW + c);
+            const int lq = wq0 + nt * 16 + r;
+            if (lq < q_len)
+                __builtin_nontemporal_store(v, reinterpret_cast<floatx4 *>(p.out + ((int64_t)(row0 + lq) * p.n_heads + head) * D + c));
+        }
+    }
+}
+
 // The staged path's launches; GLA_ERR_* when a launch fails.
 template <int D, bool Q8>
 int launch_bf16_staged(gla_ctx *ctx, const PrefillParams &prm, dim3 grid, int n_seqs, uint8_t *img, int n_tiles) {
@@ -1276,40 +1902,72 @@ int launch_bf16(gla_ctx *ctx, const PrefillParams &prm, dim3 grid) {
     return GLA_OK;
 }
 
-template <int D, int NT, int NW, bool Q8>
-int launch_f32(gla_ctx *ctx, const PrefillParams &prm, dim3 grid) {
-    if (prm.softcap > 0.0f)
-        hipLaunchKernelGGL((prefill_f32_kernel<D, NT, NW, Q8, true>), grid, dim3(NW * 64), 0, ctx->stream, prm);
-    else
-        hipLaunchKernelGGL((prefill_f32_kernel<D, NT, NW, Q8, false>), grid, dim3(NW * 64), 0, ctx->stream, prm);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "prefill_f32_kernel launch: %s", hipGetErrorString(e));
+// Tile images an fp32 prefill may hold in scratch; a call with more (sequence,
+// KV head) pairs runs in several rounds over them.
+constexpr size_t kSplitScratch = (size_t)1 << 30;
+// Query rows of a call's longest sequence up to which workgroups convert their
+// own tiles: the second launch costs a short prompt more than the repeated
+// conversion, but each row block converts the whole past again. One sequence,
+// us per call, unstaged / staged: from position 0, d = 128 20 rows 7.7 / 12.0,
+// 90 rows 12.6 / 16.1, 150 rows 17.8 / 19.7; d = 64 20 rows 5.6 / 9.2, 100 rows
+// 11.0 / 13.5; d = 256 with the soft-cap 20 rows 11.4 / 17.3, 100 rows 27.9 /
+// 30.6. After 1,000 cached positions, d = 128: 100 rows 93 / 71.
+constexpr int kUnstagedRows = 96;
+
+// fp32 prefill: the tile images of as many (sequence, KV head) pairs as the
+// scratch takes, then their attention. A call of few query blocks has each
+// workgroup convert its own tiles instead (the same bits), and so has one whose
+// scratch cannot be had: it would have to grow during a capture, the device is
+// full, or one pair's images alone pass the bound.
+template <int D, bool Q8, bool CAP>
+int launch_split(gla_ctx *ctx, PrefillParams prm, int n_pairs, int n_hgrp, int n_tiles) {
+    const size_t per = (size_t)n_tiles * (kSplitImage<D> + sizeof(TileMeta));
+    uint8_t *img = nullptr;
+    int round = n_pairs;
+    if (prm.max_q_len > kUnstagedRows && n_tiles > 0 && per <= kSplitScratch) {
+        round = (int)std::min<size_t>({(size_t)n_pairs, kSplitScratch / per, (size_t)65535});
+        void *scr = nullptr;
+        if (ensure_scratch(ctx, round * per, &scr) == GLA_OK) {
+            img = (uint8_t *)scr;
+        } else {
+            clear_error();
+            (void)hipGetLastError();
+            round = n_pairs;
+        }
+    }
+    const int rows = 16 * (img ? kSplitNT<true> : kSplitNT<false>) * (4 / prm.hpw);  // per workgroup
+    prm.n_qblocks = (prm.max_q_len + rows - 1) / rows;
+    if (prm.n_qblocks > 65535) return set_error(GLA_ERR_INVALID, "prefill: %d query blocks > 65535", prm.n_qblocks);
+    if (!img) {
+        hipLaunchKernelGGL((prefill_split_kernel<D, Q8, CAP, false>), dim3(n_pairs * n_hgrp, prm.n_qblocks), dim3(256),
+                           0, ctx->stream, prm, (const uint8_t *)nullptr, (const TileMeta *)nullptr, n_tiles, 0);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "prefill_split_kernel launch: %s", hipGetErrorString(e));
+        return GLA_OK;
+    }
+    TileMeta *meta = reinterpret_cast<TileMeta *>(img + (size_t)round * n_tiles * kSplitImage<D>);
+    for (int p0 = 0; p0 < n_pairs; p0 += round) {
+        const int np = std::min(round, n_pairs - p0);
+        hipLaunchKernelGGL((stage_split_kernel<D, Q8>), dim3(n_tiles, np), dim3(256), 0, ctx->stream, prm, img, meta,
+                           n_tiles, p0);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "stage_split_kernel launch: %s", hipGetErrorString(e));
+        hipLaunchKernelGGL((prefill_split_kernel<D, Q8, CAP, true>), dim3(np * n_hgrp, prm.n_qblocks), dim3(256), 0,
+                           ctx->stream, prm, (const uint8_t *)img, (const TileMeta *)meta, n_tiles, p0);
+        e = hipGetLastError();
+        if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "prefill_split_kernel launch: %s", hipGetErrorString(e));
+    }
     return GLA_OK;
 }
 
-// Shapes per head_dim: queries per wave (16*NT) and waves per workgroup.
-// d128 (cfg4): 4 waves of 32 queries. 8 waves of 16 queries (4 waves per
-// SIMD instead of 2) measured 4% slower: each K/V operand read from LDS then
-// feeds one MFMA instead of two.
 template <int D>
-struct PrefillShape;
-template <>
-struct PrefillShape<64> {
-    static constexpr int NT = 2, NW = 4;
-};
-template <>
-struct PrefillShape<128> {
-    static constexpr int NT = 2, NW = 4;
-};
-template <>
-struct PrefillShape<256> {
-    static constexpr int NT = 1, NW = 4;
-};
-
-template <int D>
-int launch_shape(gla_ctx *ctx, bool q8, const PrefillParams &prm, dim3 grid) {
-    using S = PrefillShape<D>;
-    return q8 ? launch_f32<D, S::NT, S::NW, true>(ctx, prm, grid) : launch_f32<D, S::NT, S::NW, false>(ctx, prm, grid);
+int launch_f32(gla_ctx *ctx, bool q8, const PrefillParams &prm, int n_pairs, int n_hgrp, int n_tiles) {
+    const bool cap = prm.softcap > 0.0f;
+    if (q8)
+        return cap ? launch_split<D, true, true>(ctx, prm, n_pairs, n_hgrp, n_tiles)
+                   : launch_split<D, true, false>(ctx, prm, n_pairs, n_hgrp, n_tiles);
+    return cap ? launch_split<D, false, true>(ctx, prm, n_pairs, n_hgrp, n_tiles)
+               : launch_split<D, false, false>(ctx, prm, n_pairs, n_hgrp, n_tiles);
 }
 
 }  // namespace
@@ -1318,20 +1976,9 @@ int launch_prefill(gla_ctx *ctx, const PrefillLaunch &a) {
     const int D = a.head_dim;
     const int group = a.n_heads / a.n_kv_heads;
     const int hpw = (group % 4 == 0) ? 4 : ((group % 2 == 0) ? 2 : 1);
-    int NT = 1, NW = 4;
-    switch (D) {
-    case 64:
-        NT = PrefillShape<64>::NT, NW = PrefillShape<64>::NW;
-        break;
-    case 128:
-        NT = PrefillShape<128>::NT, NW = PrefillShape<128>::NW;
-        break;
-    case 256:
-        NT = PrefillShape<256>::NT, NW = PrefillShape<256>::NW;
-        break;
-    default:
-        return set_error(GLA_ERR_INVALID, "unsupported head_dim %d", D);
-    }
+    if (D != 64 && D != 128 && D != 256) return set_error(GLA_ERR_INVALID, "unsupported head_dim %d", D);
+    constexpr int NT = 2;  // 32 queries per wave
+    int NW = 4;
     // bf16: the staged path keeps the bf16 tile images of every (sequence, KV
     // head) in scratch, up to 1 GiB, and its staging grid has one z row per
     // sequence (at most 65,535); beyond either each workgroup converts its own
@@ -1341,7 +1988,6 @@ int launch_prefill(gla_ctx *ctx, const PrefillLaunch &a) {
     const bool staged = a.precision == GLA_PREC_BF16 && getenv("GLA_BF16_UNSTAGED") == nullptr && n_tiles > 0 &&
                         img_bytes <= ((size_t)1 << 30) && a.n_seqs <= 65535;
     if (a.precision == GLA_PREC_BF16) {
-        NT = 2;
         if (staged)
             NW = D == 64 ? kBf16sWaves<64> : (D == 128 ? kBf16sWaves<128> : kBf16sWaves<256>);
         else
@@ -1394,13 +2040,14 @@ int launch_prefill(gla_ctx *ctx, const PrefillLaunch &a) {
             return a.q8 ? launch_bf16<256, true>(ctx, prm, grid) : launch_bf16<256, false>(ctx, prm, grid);
         }
     }
+    const int n_pairs = a.n_seqs * a.n_kv_heads, n_hgrp = group / hpw;
     switch (D) {
     case 64:
-        return launch_shape<64>(ctx, a.q8, prm, grid);
+        return launch_f32<64>(ctx, a.q8, prm, n_pairs, n_hgrp, n_tiles);
     case 128:
-        return launch_shape<128>(ctx, a.q8, prm, grid);
+        return launch_f32<128>(ctx, a.q8, prm, n_pairs, n_hgrp, n_tiles);
     default:
-        return launch_shape<256>(ctx, a.q8, prm, grid);
+        return launch_f32<256>(ctx, a.q8, prm, n_pairs, n_hgrp, n_tiles);
     }
 }
 
