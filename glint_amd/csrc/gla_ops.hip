@@ -18,13 +18,12 @@
 // (hi = f16(x * 2^s), lo = f16(x * 2^s - hi), s per vector and K slice
 // putting the slice's largest |x| near 2^14), so each block's product runs as two MFMAs with
 // exact int8 x f16 products and f32 accumulation; the f16 block scale is
-// applied in f32 per block, as the reference applies it. Each launch covers
-// up to 64 vectors, so the weights are read once per 64 vectors; K is split
-// across workgroups (the slices summed in order by each row group's last
-// workgroup to finish) so that each CU reads only its slice of the
-// activation pieces. Up to four vectors
-// take the vector-ALU kernel instead (x in f32 from LDS, no pieces). Bound:
-// HBM on the weights (34 bytes per 32 weights).
+// applied in f32 per block, as the reference applies it. Up to four vectors
+// take the vector-ALU kernel (x in f32 from LDS, no pieces), up to 64 a split-K
+// kernel, more the GEMM kernel, which shares each block pair of weights and
+// pieces through LDS; both of those round in the same order, so a vector's
+// result does not depend on the call's size. Bound: HBM on the weights (34 bytes
+// per 32 weights) for few vectors, matrix and vector issue for many.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -266,6 +265,11 @@ __device__ __forceinline__ floatx4 load_agent4(const float *p) {
                    __uint_as_float((uint32_t)(b >> 32))};
 }
 
+__device__ __forceinline__ void store_agent2(float *p, float a, float b) {
+    __hip_atomic_store(reinterpret_cast<uint64_t *>(p), (uint64_t)__float_as_uint(b) << 32 | __float_as_uint(a),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // 4 bytes x + 128 -> 4 exact f16 (1024 + byte - 1152) at o[at .. at+3].
 __device__ __forceinline__ void bytes_to_h(uint32_t u, half8 &o, int at) {
     const uint32_t lo = __builtin_amdgcn_perm(0x64646464u, u, 0x07010700u);  // bytes 0, 1 under 0x64
@@ -280,7 +284,7 @@ __device__ __forceinline__ void bytes_to_h(uint32_t u, half8 &o, int at) {
     o[at + 3] = b[1];
 }
 
-constexpr int kMaxVT = 4;        // vector tiles (16 vectors each) per launch
+constexpr int kMaxVT = 4;        // vector tiles (16 vectors each) of a call
 constexpr int kSkWaves = 4;      // waves per workgroup: a quarter of the workgroup's blocks each
 constexpr int kSkRT = 4;         // row tiles per wave (and per workgroup): 64 rows share each x fragment
 constexpr int kSkMaxSplits = 8;  // K slices per launch (summed by each row group's last workgroup)
@@ -299,8 +303,8 @@ constexpr int kSkTargetWgs = 512;
 template <int NVT>
 __global__ __launch_bounds__(kSkWaves * 64) void matvec_q8_splitk_kernel(
     const uint8_t *quants, const uint16_t *scales, int rows, int n_tiles, int n_pairs, const _Float16 *xp,
-    const float *xs, int xs_stride, int n_blocks_pad, int v0, int n_vec, int n_splits, float *out,
-    int64_t split_stride, float *y, int32_t *arrivals) {
+    const float *xs, int xs_stride, int n_blocks_pad, int n_vec, int n_splits, float *out, int64_t split_stride,
+    float *y, int32_t *arrivals) {
     constexpr int RT = kSkRT;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -314,7 +318,7 @@ __global__ __launch_bounds__(kSkWaves * 64) void matvec_q8_splitk_kernel(
     const int p1 = min(q1, p0 + per);
 
     __shared__ float xsl[NVT * 16];  // this slice's piece factors of the launch's vectors, read by the epilogue
-    if ((int)threadIdx.x < NVT * 16) xsl[threadIdx.x] = xs[(int64_t)blockIdx.y * xs_stride + v0 + threadIdx.x];
+    if ((int)threadIdx.x < NVT * 16) xsl[threadIdx.x] = xs[(int64_t)blockIdx.y * xs_stride + threadIdx.x];
 
     floatx4 acc[RT][NVT];
 #pragma unroll
@@ -326,7 +330,7 @@ __global__ __launch_bounds__(kSkWaves * 64) void matvec_q8_splitk_kernel(
     auto load_x = [&](half8 (&bh)[NVT], half8 (&bl)[NVT], int blk) {
 #pragma unroll
         for (int vt = 0; vt < NVT; vt++) {
-            const _Float16 *src = xp + (((int64_t)(v0 / 16 + vt) * n_blocks_pad + blk) * 128 + lane) * 8;
+            const _Float16 *src = xp + (((int64_t)vt * n_blocks_pad + blk) * 128 + lane) * 8;
             bh[vt] = *reinterpret_cast<const half8 *>(src);
             bl[vt] = *reinterpret_cast<const half8 *>(src + 64 * 8);
         }
@@ -421,8 +425,7 @@ __global__ __launch_bounds__(kSkWaves * 64) void matvec_q8_splitk_kernel(
 #pragma unroll
         for (int w = 1; w < kSkWaves; w++) sum += red[red_at(w, rt, vt, ln) + r];
         const int row = tile0 * 16 + rl;
-        const int v = v0 + vv;
-        if (row < rows && v < n_vec) {
+        if (row < rows && vv < n_vec) {
             if (arrivals)
                 store_agent(o + (int64_t)vv * rows + row, sum * xsl[vv]);
             else
@@ -458,14 +461,14 @@ __global__ __launch_bounds__(kSkWaves * 64) void matvec_q8_splitk_kernel(
 #pragma unroll
             for (int sl = 1; sl < kSkMaxSplits; sl++)
                 if (sl < n_splits) sum += t[k][sl];
-            if (row < rows && v0 + vv < n_vec) *reinterpret_cast<floatx4 *>(y + (int64_t)vv * rows + row) = sum;
+            if (row < rows && vv < n_vec) *reinterpret_cast<floatx4 *>(y + (int64_t)vv * rows + row) = sum;
         }
     } else {
         for (int i = threadIdx.x; i < RT * 16 * NVT * 16; i += kSkWaves * 64) {
             const int rl = i & (RT * 16 - 1);
             const int vv = i / (RT * 16);
             const int row = tile0 * 16 + rl;
-            if (row >= rows || v0 + vv >= n_vec) continue;
+            if (row >= rows || vv >= n_vec) continue;
             const int64_t at = (int64_t)vv * rows + row;
             float sum = load_agent(out + at);
             for (int sl = 1; sl < n_splits; sl++) sum += load_agent(out + sl * split_stride + at);
@@ -476,14 +479,283 @@ __global__ __launch_bounds__(kSkWaves * 64) void matvec_q8_splitk_kernel(
 
 template <int NVT>
 int launch_splitk(gla_ctx *ctx, const gla_q8w *w, const _Float16 *xp, const float *xs, int xs_stride,
-                  int n_blocks_pad, int v0, int n_vec, int n_splits, float *out, int64_t split_stride, float *y,
+                  int n_blocks_pad, int n_vec, int n_splits, float *out, int64_t split_stride, float *y,
                   int32_t *arrivals) {
     const dim3 grid((w->n_tiles + kSkRT - 1) / kSkRT, n_splits);
     hipLaunchKernelGGL((matvec_q8_splitk_kernel<NVT>), grid, dim3(kSkWaves * 64), 0, ctx->stream, w->quants,
-                       w->scales, w->rows, w->n_tiles, w->n_pairs, xp, xs, xs_stride, n_blocks_pad, v0, n_vec,
-                       n_splits, out, split_stride, y, arrivals);
+                       w->scales, w->rows, w->n_tiles, w->n_pairs, xp, xs, xs_stride, n_blocks_pad, n_vec, n_splits,
+                       out, split_stride, y, arrivals);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "matvec_q8_splitk_kernel launch: %s", hipGetErrorString(e));
+    return GLA_OK;
+}
+
+// ---- many vectors: whole K per workgroup -------------------------------------------
+
+// 16 bytes per lane from sbase + voff into LDS at m0 + 16 * lane (m0 restored).
+// The s_nop is the wait state an LDS-DMA load needs after an SALU write of M0,
+// which the compiler cannot insert into inline assembly.
+__device__ __forceinline__ void lds_copy16(const uint8_t *sbase, uint32_t voff, uint32_t m0) {
+    uint32_t save;
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %3\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %1, %2\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(save)
+        : "v"(voff), "s"(sbase), "s"(m0)
+        : "memory");
+}
+
+// 4 bytes per lane from sbase + voff into LDS at m0 + 4 * lane.
+__device__ __forceinline__ void lds_copy4(const uint8_t *sbase, uint32_t voff, uint32_t m0) {
+    uint32_t save;
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %3\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dword %1, %2\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(save)
+        : "v"(voff), "s"(sbase), "s"(m0)
+        : "memory");
+}
+
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+    static_assert(N >= 0 && N < 64, "vmcnt range");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// y[v][row] for 32*RT rows x 32*VT vectors per workgroup: the four waves are 2 x
+// 2 of RT row tiles x VT vector tiles, and each block pair of the weights, of
+// their scales and of the x pieces is copied into LDS once for all of them
+// (global_load_lds, RING - 1 pairs in flight while one is multiplied). With
+// `part` a workgroup takes the K slice blockIdx.z and the last of the tile's to
+// arrive sums the slices in order, as in the split-K kernel; without it a
+// workgroup takes all slices and no partial sum leaves it. The sums round as
+// the split-K kernel's either way: block by block into a quarter of a slice, the
+// four quarters in order, the slice times its piece factor, the slices in order.
+// Bound: with the chip full, vector and matrix issue (per block pair at 4 x 2
+// tiles 32 MFMAs, 64 scale FMAs, 64 conversions) and the copies beside them;
+// with few workgroups the 0.6 us a pair takes from its barrier to its last FMA,
+// which more pairs in flight do not shorten (6144 x 4096, 64 vectors: 41.7 us
+// with two LDS stages, 43.8 with three). 6144 x 4096, 2,048 vectors: 271 us =
+// 761 TFLOP/s of f16 products; 64 at a time in the split-K kernel 662 us.
+template <int RT, int VT, int RING>
+__global__ __launch_bounds__(256) void gemm_q8_kernel(const uint8_t *quants, const uint16_t *scales, int rows,
+                                                      int n_tiles, int n_pairs, const _Float16 *xp, const float *xs,
+                                                      int xs_stride, int n_vec_tiles, int n_vec, int n_splits,
+                                                      float *y, float *part, int64_t split_stride,
+                                                      int32_t *arrivals) {
+    constexpr int WKB = 2 * RT, XKB = 8 * VT;  // kilobytes of a pair: weights, x pieces
+    constexpr int CPW = (WKB + XKB) / 4;       // kilobyte copies per wave
+    static_assert((WKB + XKB) % 4 == 0, "copies deal evenly to the waves");
+    
+    constexpr int STAGE = (WKB + XKB + 1) * 1024;  // weights, x pieces, the weights' scales (64 bytes a tile)
+    static_assert(2 * RT <= 16, "the scales fit a kilobyte");
+    __shared__ __attribute__((aligned(16))) uint8_t lds[RING][STAGE];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kg = lane >> 4;
+    const int tile_wg = blockIdx.x * 2 * RT, vt_wg = blockIdx.y * 2 * VT;
+    const int rt0 = (wave & 1) * RT, vt0 = (wave >> 1) * VT;  // the wave's tiles in the workgroup's
+    const uint32_t ring = __builtin_amdgcn_readfirstlane(
+        (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)&lds[0][0]);
+
+    // tiles past the end re-read the last one; their sums are not stored
+    const uint8_t *src[CPW];
+    int step[CPW];  // bytes from one pair to the next
+#pragma unroll
+    for (int c = 0; c < CPW; c++) {
+        const int piece = wave * CPW + c;
+        if (piece < WKB) {
+            src[c] = quants + (int64_t)min(tile_wg + piece, n_tiles - 1) * n_pairs * 1024;
+            step[c] = 1024;
+        } else {
+            const int k = piece - WKB;  // vector tile k / 4, kilobyte k % 4 of its pair
+            src[c] = reinterpret_cast<const uint8_t *>(xp) +
+                     (int64_t)min(vt_wg + k / 4, n_vec_tiles - 1) * n_pairs * 4096 + (k & 3) * 1024;
+            step[c] = 4096;
+        }
+    }
+    // scales of four row tiles by one copy: lanes 16t .. 16t+15 take tile t's 64 bytes
+    const int stile = (wave * 4 + (lane >> 4)) % (2 * RT);
+    const uint32_t soff = (uint32_t)min(tile_wg + stile, n_tiles - 1) * (uint32_t)n_pairs * 64 + (lane & 15) * 4;
+    const uint32_t sdst = (uint32_t)(wave * 4 % (2 * RT)) * 64;
+    auto issue = [&](int p) {
+        const uint32_t dst = ring + (uint32_t)(p % RING) * STAGE;
+#pragma unroll
+        for (int c = 0; c < CPW; c++)
+            lds_copy16(src[c] + (int64_t)p * step[c], lane * 16, dst + (wave * CPW + c) * 1024);
+        lds_copy4(reinterpret_cast<const uint8_t *>(scales) + (int64_t)p * 64, soff, dst + (WKB + XKB) * 1024 + sdst);
+    };
+
+    // this workgroup's slices, and their block pairs
+    const int ps = (n_pairs + n_splits - 1) / n_splits;
+    const int s0 = part ? (int)blockIdx.z : 0, s1 = part ? s0 + 1 : n_splits;
+    const int pa = min(n_pairs, s0 * ps), pb = min(n_pairs, s1 * ps);
+    floatx4 acc[RT][VT], slice[RT][VT], total[RT][VT];
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+        for (int vt = 0; vt < VT; vt++) {
+            acc[rt][vt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            slice[rt][vt] = total[rt][vt] = acc[rt][vt];
+        }
+
+#pragma unroll
+    for (int p = 0; p < RING - 1; p++)
+        if (pa + p < pb) issue(pa + p);
+    for (int s = s0; s < s1; s++) {
+        const int q0 = min(n_pairs, s * ps), q1 = min(n_pairs, q0 + ps);
+        const int per = (q1 - q0 + kSkWaves - 1) / kSkWaves;
+        for (int w = 0; w < kSkWaves; w++) {
+            const int p1 = min(q1, q0 + (w + 1) * per);
+            for (int p = min(q1, q0 + w * per); p < p1; p++) {
+                // pair p has landed for every wave, and pair p - 1 is done with
+                if (RING == 3 && p + 1 < pb)
+                    wait_vm<CPW + 1>();
+                else
+                    wait_vm<0>();
+                __syncthreads();
+                if (p + RING - 1 < pb) issue(p + RING - 1);
+                const uint8_t *st = lds[p % RING];
+                const uint8_t *wl = st + rt0 * 1024 + lane * 16;
+                const uint8_t *xl = st + (WKB + 4 * vt0) * 1024 + lane * 16;
+                uint4 sw[RT];
+#pragma unroll
+                for (int rt = 0; rt < RT; rt++)
+                    sw[rt] = *reinterpret_cast<const uint4 *>(st + (WKB + XKB) * 1024 + (rt0 + rt) * 64 + kg * 16);
+                uint4 qw[RT];
+#pragma unroll
+                for (int rt = 0; rt < RT; rt++) qw[rt] = *reinterpret_cast<const uint4 *>(wl + rt * 1024);
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    half8 bh[VT], bl[VT];
+#pragma unroll
+                    for (int vt = 0; vt < VT; vt++) {
+                        bh[vt] = *reinterpret_cast<const half8 *>(xl + vt * 4096 + j * 2048);
+                        bl[vt] = *reinterpret_cast<const half8 *>(xl + vt * 4096 + j * 2048 + 1024);
+                    }
+#pragma unroll
+                    for (int rt = 0; rt < RT; rt++) {
+                        half8 a;
+                        bytes_to_h(j ? qw[rt].z : qw[rt].x, a, 0);
+                        bytes_to_h(j ? qw[rt].w : qw[rt].y, a, 4);
+                        // scales of rows kg*4 + r: [row][block] f16
+                        typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+                        const float sc[4] = {(float)__builtin_bit_cast(half2v, sw[rt].x)[j],
+                                             (float)__builtin_bit_cast(half2v, sw[rt].y)[j],
+                                             (float)__builtin_bit_cast(half2v, sw[rt].z)[j],
+                                             (float)__builtin_bit_cast(half2v, sw[rt].w)[j]};
+                        floatx4 c[VT];
+#pragma unroll
+                        for (int vt = 0; vt < VT; vt++)
+                            c[vt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bh[vt],
+                                                                           floatx4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+                        for (int vt = 0; vt < VT; vt++)
+                            c[vt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bl[vt], c[vt], 0, 0, 0);
+#pragma unroll
+                        for (int vt = 0; vt < VT; vt++)
+#pragma unroll
+                            for (int r = 0; r < 4; r++) acc[rt][vt][r] = fmaf(c[vt][r], sc[r], acc[rt][vt][r]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+                for (int vt = 0; vt < VT; vt++) {
+                    slice[rt][vt] = w ? slice[rt][vt] + acc[rt][vt] : acc[rt][vt];
+                    acc[rt][vt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                }
+        }
+#pragma unroll
+        for (int vt = 0; vt < VT; vt++) {
+            const int v = min(vt_wg + vt0 + vt, n_vec_tiles - 1) * 16 + (lane & 15);
+            const float f = xs[(int64_t)s * xs_stride + v];
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++) {
+                const floatx4 t = slice[rt][vt] * f;  // f is a power of two
+                total[rt][vt] = s > s0 ? total[rt][vt] + t : t;
+            }
+        }
+    }
+
+    // the lane's outputs: of vector (vt_wg + vt0 + vt)*16 + lane % 16 the rows
+    // (tile_wg + rt0 + rt)*16 + 4*kg .. +3
+    const bool quads = rows % 4 == 0 && ((uintptr_t)y & 15) == 0;
+    const auto each = [&](auto f) {
+#pragma unroll
+        for (int vt = 0; vt < VT; vt++) {
+            const int v = (vt_wg + vt0 + vt) * 16 + (lane & 15);
+            if (v >= n_vec) continue;
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++) {
+                const int row = (tile_wg + rt0 + rt) * 16 + kg * 4;
+                if (row < rows) f((int64_t)v * rows + row, rows - row, total[rt][vt]);
+            }
+        }
+    };
+    if (part) {
+        float *o = part + s0 * split_stride;
+        each([&](int64_t at, int left, const floatx4 &t) {
+            if (quads) {
+                store_agent2(o + at, t[0], t[1]);
+                store_agent2(o + at + 2, t[2], t[3]);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (r < left) store_agent(o + at + r, t[r]);
+            }
+        });
+        __shared__ int last;
+        if (!arrive_last(arrivals + blockIdx.y * gridDim.x + blockIdx.x, n_splits, &last)) return;
+        each([&](int64_t at, int left, floatx4 &t) {
+            floatx4 got[kSkMaxSplits];
+#pragma unroll
+            for (int s = 0; s < kSkMaxSplits; s++)
+                if (s < n_splits) {
+                    if (quads) {
+                        got[s] = load_agent4(part + s * split_stride + at);
+                    } else {
+#pragma unroll
+                        for (int r = 0; r < 4; r++) got[s][r] = r < left ? load_agent(part + s * split_stride + at + r) : 0.0f;
+                    }
+                }
+            t = got[0];
+#pragma unroll
+            for (int s = 1; s < kSkMaxSplits; s++)
+                if (s < n_splits) t += got[s];
+        });
+    }
+    each([&](int64_t at, int left, const floatx4 &t) {
+        if (quads) {
+            *reinterpret_cast<floatx4 *>(y + at) = t;
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (r < left) y[at + r] = t[r];
+        }
+    });
+}
+
+template <int RT, int VT, int RING>
+int launch_gemm(gla_ctx *ctx, const gla_q8w *w, const _Float16 *xp, const float *xs, int xs_stride, int n_vec,
+                int n_splits, float *y, float *part) {
+    const int n_vec_tiles = (n_vec + 15) / 16;
+    const dim3 grid((w->n_tiles + 2 * RT - 1) / (2 * RT), (n_vec_tiles + 2 * VT - 1) / (2 * VT), part ? n_splits : 1);
+    int32_t *arrivals = nullptr;
+    if (part)
+        if (int rc = ensure_arrivals(ctx, (size_t)grid.x * grid.y, &arrivals)) return rc;
+    hipLaunchKernelGGL((gemm_q8_kernel<RT, VT, RING>), grid, dim3(256), 0, ctx->stream, w->quants, w->scales, w->rows,
+                       w->n_tiles, w->n_pairs, xp, xs, xs_stride, n_vec_tiles, n_vec, n_splits, y, part,
+                       (int64_t)n_vec * w->rows, arrivals);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "gemm_q8_kernel launch: %s", hipGetErrorString(e));
     return GLA_OK;
 }
 
@@ -822,8 +1094,29 @@ int gla_matvec_q8_0(gla_ctx *ctx, const gla_q8w *w, const float *x, int n_vec, f
     const size_t xp_bytes = (size_t)vec_pad * n_blocks_pad * 32 * 2 * sizeof(_Float16);  // hi + lo per element
     const int ps = (w->n_pairs + n_splits - 1) / n_splits;  // block pairs per slice, as the split-K kernel takes them
     const size_t xs_bytes = ((size_t)n_splits * vec_pad * sizeof(float) + 255) / 256 * 256;  // [slice][vector]
-    const int64_t split_stride = (int64_t)16 * kMaxVT * w->rows;  // one slice of partials: 64 vectors x rows
-    const size_t part_bytes = n_splits > 1 ? (size_t)n_splits * split_stride * sizeof(float) : 0;
+    // Up to 64 vectors the split-K kernel, which reads every weight once and
+    // keeps more of them in flight (6144 x 4096 from HBM, 64 vectors: 25.0 us
+    // per call against 28.5); above them the GEMM kernel. Its workgroups each
+    // walk all of K where they are many enough; where they are few and K is
+    // long, they take one K slice each, unless the partial sums cost more than
+    // that saves. us per call, whole K (2 x 2 tiles) / sliced: 6144 x 4096 100
+    // vectors 42.8 / 35.0, 200 54.0 / 53.0 (25 MB of partials), 400 75.1 / 90.4
+    // (49 MB); 4096 x 4096 200 47.4 / 43.1 (26 MB), 400 60.4 / 72.4 (52 MB);
+    // 1024 x 4096 400 48.9 / 32.9 (13 MB), 997 51.3 / 58.0 (33 MB); 576 x 576
+    // 100 11.1 / 11.4. The split-K kernel, 64 vectors at a time, takes 41.3,
+    // 77.2, 140; 71.5, 128; 105, 238; 21.0.
+    constexpr size_t kMaxSliceBytes = (size_t)28 << 20;
+    constexpr int kMinSlicePairs = 32;
+    const bool few_tiles = n_vec <= 16 * kMaxVT;
+    const auto gemm_tiles = [&](int rt, int vt) {
+        return (int64_t)((w->n_tiles + 2 * rt - 1) / (2 * rt)) * ((vec_pad / 16 + 2 * vt - 1) / (2 * vt));
+    };
+    const int64_t split_stride = (int64_t)n_vec * w->rows;  // one slice of partials
+    size_t part_bytes = n_splits > 1 ? (size_t)n_splits * split_stride * sizeof(float) : 0;
+    // (4 x 2 tiles on two workgroups per CU: 6144 x 4096 2,048 vectors 271 us, 2 x 2 tiles 281)
+    const bool sliced = !few_tiles && n_splits > 1 && w->n_pairs >= kMinSlicePairs && part_bytes <= kMaxSliceBytes &&
+                        gemm_tiles(4, 2) < 512;
+    if (!few_tiles && !sliced) part_bytes = 0;
     void *scr = nullptr;
     int rc = ensure_scratch(ctx, xp_bytes + xs_bytes + part_bytes, &scr);
     if (rc != GLA_OK) return rc;
@@ -839,36 +1132,29 @@ int gla_matvec_q8_0(gla_ctx *ctx, const gla_q8w *w, const float *x, int n_vec, f
                            n_blocks_pad, ps, vec_pad, xp, xs);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "split_x_kernel launch: %s", hipGetErrorString(e));
-    // K slices summed in the split-K kernel by each row group's last workgroup
-    int32_t *arrivals = nullptr;
-    if (n_splits > 1) {
-        rc = ensure_arrivals(ctx, (size_t)n_groups, &arrivals);
-        if (rc != GLA_OK) return rc;
-    }
-    for (int v0 = 0; v0 < n_vec; v0 += 16 * kMaxVT) {
-        const int nvt = std::min(kMaxVT, (n_vec - v0 + 15) / 16);
-        float *yv = y + (int64_t)v0 * w->rows;
-        float *out = n_splits > 1 ? part : yv;
-        switch (nvt) {
-        case 1:
-            rc = launch_splitk<1>(ctx, w, xp, xs, vec_pad, n_blocks_pad, v0, n_vec, n_splits, out, split_stride, yv,
-                                 arrivals);
-            break;
-        case 2:
-            rc = launch_splitk<2>(ctx, w, xp, xs, vec_pad, n_blocks_pad, v0, n_vec, n_splits, out, split_stride, yv,
-                                 arrivals);
-            break;
-        case 3:
-            rc = launch_splitk<3>(ctx, w, xp, xs, vec_pad, n_blocks_pad, v0, n_vec, n_splits, out, split_stride, yv,
-                                 arrivals);
-            break;
-        default:
-            rc = launch_splitk<4>(ctx, w, xp, xs, vec_pad, n_blocks_pad, v0, n_vec, n_splits, out, split_stride, yv,
-                                 arrivals);
+    if (few_tiles) {
+        // K slices summed in the split-K kernel by each row group's last workgroup
+        int32_t *arrivals = nullptr;
+        if (n_splits > 1) {
+            rc = ensure_arrivals(ctx, (size_t)n_groups, &arrivals);
+            if (rc != GLA_OK) return rc;
         }
-        if (rc != GLA_OK) return rc;
+        float *out = n_splits > 1 ? part : y;
+        switch (vec_pad / 16) {
+        case 1:
+            return launch_splitk<1>(ctx, w, xp, xs, vec_pad, n_blocks_pad, n_vec, n_splits, out, split_stride, y, arrivals);
+        case 2:
+            return launch_splitk<2>(ctx, w, xp, xs, vec_pad, n_blocks_pad, n_vec, n_splits, out, split_stride, y, arrivals);
+        case 3:
+            return launch_splitk<3>(ctx, w, xp, xs, vec_pad, n_blocks_pad, n_vec, n_splits, out, split_stride, y, arrivals);
+        default:
+            return launch_splitk<4>(ctx, w, xp, xs, vec_pad, n_blocks_pad, n_vec, n_splits, out, split_stride, y, arrivals);
+        }
     }
-    return GLA_OK;
+    if (sliced) return launch_gemm<2, 1, 3>(ctx, w, xp, xs, vec_pad, n_vec, n_splits, y, part);
+    if (gemm_tiles(4, 2) >= 512) return launch_gemm<4, 2, 3>(ctx, w, xp, xs, vec_pad, n_vec, n_splits, y, nullptr);
+    if (gemm_tiles(2, 2) >= 128) return launch_gemm<2, 2, 2>(ctx, w, xp, xs, vec_pad, n_vec, n_splits, y, nullptr);
+    return launch_gemm<2, 1, 2>(ctx, w, xp, xs, vec_pad, n_vec, n_splits, y, nullptr);
 }
 
 int gla_q8w_rows(const gla_q8w *w) { return w ? w->rows : -1; }

@@ -203,3 +203,28 @@ def test_ops_argument_errors_and_empty_calls(backend):
     with pytest.raises(GlaError) as e:
         _rope_gpu(backend, x, [5, 9], 0, 10000.0, 1.0, 8)  # head_dim 0
     assert e.value.code == GLA_ERR_INVALID
+
+
+@pytest.mark.parametrize("rows,cols,n_vec", [
+    (193, 4096, 65),    # K slices, odd rows: scalar partials and stores
+    (192, 4096, 100),   # K slices, whole row quads
+    (100, 96, 80),      # one K slice, 2 x 1 tiles
+    (576, 576, 1000),   # whole K, 2 x 2 tiles
+    (575, 576, 997),    # the same with odd rows and a part-filled last vector tile
+    (2048, 64, 2047),   # whole K, 4 x 2 tiles and three LDS stages, a single block pair
+    (2000, 224, 2048),  # the same over an odd number of blocks
+])
+def test_matvec_q8_0_many_vectors(backend, rows, cols, n_vec):
+    """The GEMM kernel's variants: every vector has the bits of a 16-vector call (the split-K kernel), and
+    the f64 product of the dequantised rows within 2e-6 of sum |x w|."""
+    raw = orc.q8_quantize_rows(synth.normal_rows(901, rows, cols)).reshape(-1)
+    x = synth.normal(902, (n_vec, cols))
+    got = _matvec_gpu(backend, raw, rows, cols, x)
+    for v0 in sorted({0, n_vec // 2, n_vec - 16}):
+        sixteen = _matvec_gpu(backend, raw, rows, cols, x[v0:v0 + 16])
+        assert np.array_equal(got[v0:v0 + 16].view(np.uint32), sixteen.view(np.uint32)), v0
+    blk = raw.reshape(rows, cols // 32, 34)
+    w = blk[..., 2:].view(np.int8).astype(np.float64) * blk[..., :2].copy().view(np.float16).astype(np.float64)
+    w = w.reshape(rows, cols)
+    err = np.abs(got - x.astype(np.float64) @ w.T)
+    assert np.all(err <= 2e-6 * (np.abs(x).astype(np.float64) @ np.abs(w).T) + 1e-30)
