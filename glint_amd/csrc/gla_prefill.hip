@@ -1069,10 +1069,10 @@ constexpr int kCopiesPerWave = D == 64 ? 2 : (D == 128 ? 4 : 8);
 template <int D>
 constexpr int kBf16sOccupancy = D == 64 ? 4 : (D == 128 ? 3 : 1);
 
-template <int D, bool CAP>
+template <int D, bool CAP, int NT>
 __global__ __launch_bounds__(kBf16sWaves<D> * 64, kBf16sOccupancy<D>) void prefill_bf16s_kernel(const PrefillParams p,
                                                                           const uint8_t *img, int n_tiles) {
-    constexpr int NW = kBf16sWaves<D>, NT = 2;
+    constexpr int NW = kBf16sWaves<D>;
     constexpr int QW = 16 * NT;
     constexpr int KS = D / 32;
     constexpr int DT = D / 16;
@@ -1561,17 +1561,13 @@ __global__ __launch_bounds__(256) void stage_split_kernel(const PrefillParams p,
 // d = 256, whose registers are full).
 template <int D, bool STAGED>
 constexpr int kSplitOccupancy = !STAGED ? (D == 64 ? 2 : 1) : (D == 64 ? 3 : (D == 128 ? 2 : 1));
-// 16-query tiles per wave: two share every operand read; the few rows of an
-// unstaged call are spread over more waves instead.
-template <bool STAGED>
-constexpr int kSplitNT = STAGED ? 2 : 1;
 
-template <int D, bool Q8, bool CAP, bool STAGED>
+template <int D, bool Q8, bool CAP, bool STAGED, int NT>
 __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED>)) void prefill_split_kernel(const PrefillParams p,
                                                                                 const uint8_t *img,
                                                                                 const TileMeta *meta, int n_tiles,
                                                                                 int pair0) {
-    constexpr int NW = 4, NT = kSplitNT<STAGED>;
+    constexpr int NW = 4;
     constexpr int QW = 16 * NT;
     constexpr int KS = D / 32;
     constexpr int DT = D / 16;
@@ -1873,19 +1869,44 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED>)) void prefill_spl
     }
 }
 
-// The staged path's launches; GLA_ERR_* when a launch fails.
+// Query blocks of a call whose waves (four to a workgroup) take nt 16-query
+// tiles each.
+int wg_blocks(const PrefillParams &prm, int nt) {
+    const int rows = 16 * nt * (4 / prm.hpw);
+    return (prm.max_q_len + rows - 1) / rows;
+}
+// 16-query tiles per wave of a staged kernel: two share every operand read, one
+// gives twice the workgroups (the same bits), which is worth more until they
+// fill the chip: at up to 1.5 workgroups per CU. us per call, two tiles / one,
+// 32/8 heads, d = 128: 400 rows (104 workgroups of two tiles) f32 32.5 / 25.0,
+// bf16 18.6 / 14.4; 1,500 rows (376) 97.9 / 78.4, 47.5 / 39.6; 2 x 1,000 rows
+// (512) 76.6 / 72.7, 39.4 / 40.9; 217 rows after 3,800 cached, Q8_0, bf16 104.7 /
+// 76.5; six Gemma-2 prompts (528, half of them empty) f32 96.2 / 104.9.
+int wave_tiles(const gla_ctx *ctx, const PrefillParams &prm, int n_units) {
+    return 2 * (int64_t)n_units * wg_blocks(prm, 2) <= 3 * (int64_t)ctx->n_cu ? 1 : 2;
+}
+
+template <int D, bool CAP>
+void launch_bf16s(gla_ctx *ctx, PrefillParams prm, int n_units, const uint8_t *img, int n_tiles) {
+    const int nt = wave_tiles(ctx, prm, n_units);
+    prm.n_qblocks = wg_blocks(prm, nt);
+    const dim3 grid(n_units, prm.n_qblocks), block(kBf16sWaves<D> * 64);
+    if (nt == 1)
+        hipLaunchKernelGGL((prefill_bf16s_kernel<D, CAP, 1>), grid, block, 0, ctx->stream, prm, img, n_tiles);
+    else
+        hipLaunchKernelGGL((prefill_bf16s_kernel<D, CAP, 2>), grid, block, 0, ctx->stream, prm, img, n_tiles);
+}
+
 template <int D, bool Q8>
-int launch_bf16_staged(gla_ctx *ctx, const PrefillParams &prm, dim3 grid, int n_seqs, uint8_t *img, int n_tiles) {
+int launch_bf16_staged(gla_ctx *ctx, const PrefillParams &prm, int n_units, int n_seqs, uint8_t *img, int n_tiles) {
     hipLaunchKernelGGL((stage_bf16_kernel<D, Q8>), dim3(n_tiles, prm.n_kv_heads, n_seqs), dim3(256), 0, ctx->stream,
                        prm, img, n_tiles);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "stage_bf16_kernel launch: %s", hipGetErrorString(e));
     if (prm.softcap > 0.0f)
-        hipLaunchKernelGGL((prefill_bf16s_kernel<D, true>), grid, dim3(kBf16sWaves<D> * 64), 0, ctx->stream, prm,
-                           (const uint8_t *)img, n_tiles);
+        launch_bf16s<D, true>(ctx, prm, n_units, img, n_tiles);
     else
-        hipLaunchKernelGGL((prefill_bf16s_kernel<D, false>), grid, dim3(kBf16sWaves<D> * 64), 0, ctx->stream, prm,
-                           (const uint8_t *)img, n_tiles);
+        launch_bf16s<D, false>(ctx, prm, n_units, img, n_tiles);
     e = hipGetLastError();
     if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "prefill_bf16s_kernel launch: %s", hipGetErrorString(e));
     return GLA_OK;
@@ -1935,11 +1956,12 @@ int launch_split(gla_ctx *ctx, PrefillParams prm, int n_pairs, int n_hgrp, int n
             round = n_pairs;
         }
     }
-    const int rows = 16 * (img ? kSplitNT<true> : kSplitNT<false>) * (4 / prm.hpw);  // per workgroup
-    prm.n_qblocks = (prm.max_q_len + rows - 1) / rows;
+    // (the few rows of an unstaged call are spread over the most waves)
+    const int nt = img ? wave_tiles(ctx, prm, std::min(round, n_pairs) * n_hgrp) : 1;
+    prm.n_qblocks = wg_blocks(prm, nt);
     if (prm.n_qblocks > 65535) return set_error(GLA_ERR_INVALID, "prefill: %d query blocks > 65535", prm.n_qblocks);
     if (!img) {
-        hipLaunchKernelGGL((prefill_split_kernel<D, Q8, CAP, false>), dim3(n_pairs * n_hgrp, prm.n_qblocks), dim3(256),
+        hipLaunchKernelGGL((prefill_split_kernel<D, Q8, CAP, false, 1>), dim3(n_pairs * n_hgrp, prm.n_qblocks), dim3(256),
                            0, ctx->stream, prm, (const uint8_t *)nullptr, (const TileMeta *)nullptr, n_tiles, 0);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "prefill_split_kernel launch: %s", hipGetErrorString(e));
@@ -1952,8 +1974,13 @@ int launch_split(gla_ctx *ctx, PrefillParams prm, int n_pairs, int n_hgrp, int n
                            n_tiles, p0);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "stage_split_kernel launch: %s", hipGetErrorString(e));
-        hipLaunchKernelGGL((prefill_split_kernel<D, Q8, CAP, true>), dim3(np * n_hgrp, prm.n_qblocks), dim3(256), 0,
-                           ctx->stream, prm, (const uint8_t *)img, (const TileMeta *)meta, n_tiles, p0);
+        const dim3 grid(np * n_hgrp, prm.n_qblocks);
+        if (nt == 1)
+            hipLaunchKernelGGL((prefill_split_kernel<D, Q8, CAP, true, 1>), grid, dim3(256), 0, ctx->stream, prm,
+                               (const uint8_t *)img, (const TileMeta *)meta, n_tiles, p0);
+        else
+            hipLaunchKernelGGL((prefill_split_kernel<D, Q8, CAP, true, 2>), grid, dim3(256), 0, ctx->stream, prm,
+                               (const uint8_t *)img, (const TileMeta *)meta, n_tiles, p0);
         e = hipGetLastError();
         if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "prefill_split_kernel launch: %s", hipGetErrorString(e));
     }
@@ -2021,14 +2048,14 @@ int launch_prefill(gla_ctx *ctx, const PrefillLaunch &a) {
             uint8_t *img = (uint8_t *)scr;
             switch (D) {
             case 64:
-                return a.q8 ? launch_bf16_staged<64, true>(ctx, prm, grid, a.n_seqs, img, n_tiles)
-                            : launch_bf16_staged<64, false>(ctx, prm, grid, a.n_seqs, img, n_tiles);
+                return a.q8 ? launch_bf16_staged<64, true>(ctx, prm, grid.x, a.n_seqs, img, n_tiles)
+                            : launch_bf16_staged<64, false>(ctx, prm, grid.x, a.n_seqs, img, n_tiles);
             case 128:
-                return a.q8 ? launch_bf16_staged<128, true>(ctx, prm, grid, a.n_seqs, img, n_tiles)
-                            : launch_bf16_staged<128, false>(ctx, prm, grid, a.n_seqs, img, n_tiles);
+                return a.q8 ? launch_bf16_staged<128, true>(ctx, prm, grid.x, a.n_seqs, img, n_tiles)
+                            : launch_bf16_staged<128, false>(ctx, prm, grid.x, a.n_seqs, img, n_tiles);
             default:
-                return a.q8 ? launch_bf16_staged<256, true>(ctx, prm, grid, a.n_seqs, img, n_tiles)
-                            : launch_bf16_staged<256, false>(ctx, prm, grid, a.n_seqs, img, n_tiles);
+                return a.q8 ? launch_bf16_staged<256, true>(ctx, prm, grid.x, a.n_seqs, img, n_tiles)
+                            : launch_bf16_staged<256, false>(ctx, prm, grid.x, a.n_seqs, img, n_tiles);
             }
         }
         switch (D) {

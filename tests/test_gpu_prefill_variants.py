@@ -1,5 +1,6 @@
-"""fp32 prefill on split f16 pieces: staged and unstaged tiles, what the pieces cannot carry, calls
-whose scratch cannot be had, and calls whose tile images take several rounds."""
+"""Prefill's kernel variants: fp32 on split f16 pieces (staged and unstaged tiles, what the pieces cannot
+carry, calls whose scratch cannot be had or whose tile images take several rounds), and one or two query
+tiles per wave (both precisions)."""
 from __future__ import annotations
 
 import numpy as np
@@ -32,6 +33,23 @@ def test_staged_equals_unstaged(backend, dtype, d, H, Hkv):
         few = len(lens) - 1
         alone = run_prefill(backend, c.cache, q[:start[few]], start[:few + 1], offs[:few], H, 0.1, cap, window)
         assert np.array_equal(_bits(alone), _bits(both[:start[few]])), (dtype, d, cap, window)
+
+
+@pytest.mark.parametrize("precision", ["f32", "bf16"])
+@pytest.mark.parametrize("d,H,Hkv,rows", [(64, 8, 2, 900), (128, 8, 2, 900), (256, 4, 2, 1700)])
+def test_one_and_two_query_tiles_per_wave(backend, precision, d, H, Hkv, rows):
+    """A call that fills the chip gives each wave two 16-query tiles, a smaller one (here the same prompts
+    alone, a part-filled last tile included) one: the same bits."""
+    lens = [rows, rows - 13, 200, rows, rows, rows, rows, rows]
+    c = Contig(backend, "f32", len(lens), 1, rows, Hkv, d, seed=3300 + d)
+    q = synth.normal(3400 + d, (sum(lens), H, d))
+    start = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    both = run_prefill(backend, c.cache, q, start, [0] * len(lens), H, 0.1, None, 333, precision=precision)
+    for b in (0, 1, 2):
+        part = slice(start[b], start[b + 1])
+        alone = run_prefill(backend, c.cache, q[part], [0, lens[b]], [0], H, 0.1, None, 333, precision=precision,
+                            seq_slot=np.array([b], np.int32))
+        assert np.array_equal(_bits(alone), _bits(both[part])), (precision, d, b)
 
 
 # (K row, V column, q row) multipliers of the values that leave the pieces' range, one at a time, and with
