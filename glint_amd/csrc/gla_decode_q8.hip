@@ -795,6 +795,18 @@ __device__ __forceinline__ void wave_chunk(const Q8Params &p, const Range &r, in
     }
 }
 
+// Pages per workgroup of a window of n pages: `full`, but a window of two
+// workgroups is cut in half, so that neither walks longer than it has to. Four
+// sequences of 200-2,000 positions at 32/8 heads, d = 128 (125 pages: 112 + 13
+// before): 25.6 -> 20.6 us per call, 16 of 1,900-2,500 66 -> 56, 64 of
+// 128-8,192 96.2 -> 95.2. Windows of three workgroups and more keep full ones:
+// cut evenly, the last batch takes 96.1, and so does head_dim 256 (32 Gemma-2 sequences of 2,048-8,192, a
+// window and a global layer: 199.6 -> 214.6). A rule on the window alone, as
+// batch invariance needs.
+__host__ __device__ __forceinline__ int wg_span(int n, int full, int D) {
+    return D <= 128 && n > full && n <= 2 * full ? ((n + 1) / 2 + 1) & ~1 : full;
+}
+
 // One workgroup item: (sequence b, its workgroup wg, KV head x head group hx).
 // The 4 waves take 4 consecutive chunks of the unit and merge them in LDS; a
 // unit longer than one workgroup writes one partial per workgroup.
@@ -822,7 +834,7 @@ __device__ __forceinline__ void q8_item(const Q8Params &p, uint8_t (*slots)[kSlo
     // left) and splits them evenly over its waves, so the waves of the
     // sequence's last, short workgroup finish together instead of one wave
     // working while the others wait at the merge.
-    const int span = kWaves * p.ch;
+    const int span = wg_span(r.n_pages, kWaves * p.ch, D);
     // (at most max_wg: partial slots are sized from the host lengths, and a
     // caller whose host copies disagree with the device arrays gets a wrong
     // result, never an access outside the slots)
@@ -946,7 +958,7 @@ __global__ __launch_bounds__(kGT * D / 4) void decode_q8_combine_kernel(const Q8
     const int gcount = min(p.hpw, p.group - g0);
     const int h_base = kvh * p.group + g0;
     const Range r = seq_range(p, b);
-    const int span = kWaves * p.ch;  // pages per workgroup
+    const int span = wg_span(r.n_pages, kWaves * p.ch, D);  // pages per workgroup
     const int n_wg = min((r.n_pages + span - 1) / span, p.max_wg);
     if (n_wg <= 1) return;
     const int g = (4 * (int)threadIdx.x) / D;
@@ -1083,11 +1095,11 @@ int launch_decode_q8(gla_ctx *ctx, const DecodeLaunch &d) {
         const int v = atoi(env);
         if (v > 0) ch = std::min(64, (v + 1) & ~1);
     }
-    const int span = kWaves * ch;  // pages per workgroup
+    const int full = kWaves * ch;  // pages per workgroup, at most
     // workgroups per unit: exact with host lengths, else the max_kv_len bound
     int64_t max_wg = 1, wg_total = 0;
     for (int b = 0; b < d.n_seqs; b++) {
-        const int64_t nw = ((int64_t)pages_of(b) + span - 1) / span;
+        const int64_t nw = ((int64_t)pages_of(b) + full - 1) / full;
         max_wg = std::max(max_wg, nw);
         wg_total += std::max<int64_t>(nw, 1);
     }
@@ -1140,21 +1152,21 @@ int launch_decode_q8(gla_ctx *ctx, const DecodeLaunch &d) {
     // counts (0 .. span) keeps the order stable and allocates nothing.
     prm.n_rows = 0;
     if (host && max_wg <= 64 && d.n_seqs <= 1024 && wg_total <= kMaxRows) {
-        int count[4 * 64 + 2] = {0};  // rows per page count, span <= 256
-        auto wg_pages = [&](int n, int j) { return n == 0 ? 0 : std::min(span, n - j * span); };
+        int count[4 * 64 + 2] = {0};  // rows per page count, full <= 256
+        auto wg_pages = [&](int n, int j, int span) { return n == 0 ? 0 : std::min(span, n - j * span); };
         for (int b = 0; b < d.n_seqs; b++) {
-            const int n = pages_of(b);
-            for (int j = 0; j == 0 || j * span < n; j++) count[wg_pages(n, j)]++;
+            const int n = pages_of(b), span = wg_span(n, full, D);
+            for (int j = 0; j == 0 || j * span < n; j++) count[wg_pages(n, j, span)]++;
         }
         int at[4 * 64 + 2];  // first row of each page count, longest first
         int next = 0;
-        for (int c = span; c >= 0; c--) {
+        for (int c = full; c >= 0; c--) {
             at[c] = next;
             next += count[c];
         }
         for (int b = 0; b < d.n_seqs; b++) {
-            const int n = pages_of(b);
-            for (int j = 0; j == 0 || j * span < n; j++) prm.rows[at[wg_pages(n, j)]++] = (uint16_t)(b << 6 | j);
+            const int n = pages_of(b), span = wg_span(n, full, D);
+            for (int j = 0; j == 0 || j * span < n; j++) prm.rows[at[wg_pages(n, j, span)]++] = (uint16_t)(b << 6 | j);
         }
         prm.n_rows = next;
         grid = dim3(d.n_kv_heads * n_hg, (unsigned)next, 1);

@@ -352,3 +352,28 @@ def test_host_lengths_outside_the_storage_are_refused(backend, dtype):
     want = _oracle_decode(p.stores, q, pb.kv_start, pb.kv_len, H, Hkv, d, 0.125)
     got = run_decode(backend, p.pool, q, pb.kv_start, pb.kv_len, H, 0.125, table=pb.table)
     assert_close(got, want, what=f"{dtype} after the refusals")
+
+
+@pytest.mark.parametrize("d,full", [(64, 112), (128, 112), (256, 160)])
+def test_q8_windows_of_one_two_and_three_workgroups(backend, d, full):
+    """Q8_0 windows on both sides of one and of two workgroups (`full` pages each; two share their window
+    evenly up to d = 128), from a page boundary and from inside a page: against the oracle, and the same
+    bits alone, without host lengths and in a batch."""
+    H, Hkv = 8, 2
+    pages = [full - 1, full, full + 1, full + 2, 2 * full - 1, 2 * full, 2 * full + 1]
+    lens = np.array([16 * n for n in pages] + [16 * full + 1, 16 * full], np.int32)
+    starts = np.array([0] * len(pages) + [0, 7], np.int32)  # the last: `full` pages' positions over full + 1 pages
+    max_seq = int((starts + lens).max())
+    c = Contig(backend, "q8", 1, 1, max_seq, Hkv, d, seed=7100 + d)
+    B = len(lens)
+    q = synth.normal(7200 + d, (B, H, d))
+    slot = np.zeros(B, np.int32)
+    scale = 1 / np.sqrt(d)
+    got = run_decode(backend, c.cache, q, starts, lens, H, scale, seq_slot=slot)
+    bare = run_decode(backend, c.cache, q, starts, lens, H, scale, seq_slot=slot, host_lengths=False)
+    assert np.array_equal(got.view(np.uint32), bare.view(np.uint32))
+    want = orc.decode_batch(q.reshape(B, H * d), [c.stores[0]] * B, 0, starts, lens, H, Hkv, d, scale, None).reshape(B, H, d)
+    assert_close(got, want, what=f"d{d}")
+    for b in range(B):
+        alone = run_decode(backend, c.cache, q[b:b + 1], starts[b:b + 1], lens[b:b + 1], H, scale, seq_slot=slot[:1])
+        assert np.array_equal(alone.view(np.uint32), got[b:b + 1].view(np.uint32)), b
