@@ -745,12 +745,9 @@ __global__ __launch_bounds__(256) void gemm_q8_kernel(const uint8_t *quants, con
 
 template <int RT, int VT, int RING>
 int launch_gemm(gla_ctx *ctx, const gla_q8w *w, const _Float16 *xp, const float *xs, int xs_stride, int n_vec,
-                int n_splits, float *y, float *part) {
+                int n_splits, float *y, float *part, int32_t *arrivals) {
     const int n_vec_tiles = (n_vec + 15) / 16;
     const dim3 grid((w->n_tiles + 2 * RT - 1) / (2 * RT), (n_vec_tiles + 2 * VT - 1) / (2 * VT), part ? n_splits : 1);
-    int32_t *arrivals = nullptr;
-    if (part)
-        if (int rc = ensure_arrivals(ctx, (size_t)grid.x * grid.y, &arrivals)) return rc;
     hipLaunchKernelGGL((gemm_q8_kernel<RT, VT, RING>), grid, dim3(256), 0, ctx->stream, w->quants, w->scales, w->rows,
                        w->n_tiles, w->n_pairs, xp, xs, xs_stride, n_vec_tiles, n_vec, n_splits, y, part,
                        (int64_t)n_vec * w->rows, arrivals);
@@ -1112,14 +1109,30 @@ int gla_matvec_q8_0(gla_ctx *ctx, const gla_q8w *w, const float *x, int n_vec, f
         return (int64_t)((w->n_tiles + 2 * rt - 1) / (2 * rt)) * ((vec_pad / 16 + 2 * vt - 1) / (2 * vt));
     };
     const int64_t split_stride = (int64_t)n_vec * w->rows;  // one slice of partials
-    size_t part_bytes = n_splits > 1 ? (size_t)n_splits * split_stride * sizeof(float) : 0;
+    const size_t part_bytes = (size_t)n_splits * split_stride * sizeof(float);
     // (4 x 2 tiles on two workgroups per CU: 6144 x 4096 2,048 vectors 271 us, 2 x 2 tiles 281)
-    const bool sliced = !few_tiles && n_splits > 1 && w->n_pairs >= kMinSlicePairs && part_bytes <= kMaxSliceBytes &&
-                        gemm_tiles(4, 2) < 512;
-    if (!few_tiles && !sliced) part_bytes = 0;
+    bool sliced = !few_tiles && n_splits > 1 && w->n_pairs >= kMinSlicePairs && part_bytes <= kMaxSliceBytes &&
+                  gemm_tiles(4, 2) < 512;
+    // Every eager call leaves scratch and counters for 64 vectors' slices, so
+    // that a captured call of up to 64 finds them after a longer eager one. A
+    // sliced call whose own partials or counters cannot be had (they would have
+    // to grow during a capture, or the device is full) walks all of K: the same bits.
+    const size_t base_part = n_splits > 1 ? (size_t)n_splits * 16 * kMaxVT * w->rows * sizeof(float) : 0;
     void *scr = nullptr;
-    int rc = ensure_scratch(ctx, xp_bytes + xs_bytes + part_bytes, &scr);
-    if (rc != GLA_OK) return rc;
+    int32_t *arrivals = nullptr;
+    if (sliced) {
+        if (ensure_scratch(ctx, xp_bytes + xs_bytes + std::max(part_bytes, base_part), &scr) != GLA_OK ||
+            ensure_arrivals(ctx, std::max<size_t>(gemm_tiles(2, 1), n_groups), &arrivals) != GLA_OK) {
+            clear_error();
+            (void)hipGetLastError();
+            sliced = false;
+        }
+    }
+    if (!sliced) {
+        int rc = ensure_scratch(ctx, xp_bytes + xs_bytes + base_part, &scr);
+        if (rc == GLA_OK && n_splits > 1) rc = ensure_arrivals(ctx, (size_t)n_groups, &arrivals);
+        if (rc != GLA_OK) return rc;
+    }
     _Float16 *xp = (_Float16 *)scr;
     float *xs = (float *)((uint8_t *)scr + xp_bytes);
     float *part = (float *)((uint8_t *)scr + xp_bytes + xs_bytes);
@@ -1134,11 +1147,6 @@ int gla_matvec_q8_0(gla_ctx *ctx, const gla_q8w *w, const float *x, int n_vec, f
     if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "split_x_kernel launch: %s", hipGetErrorString(e));
     if (few_tiles) {
         // K slices summed in the split-K kernel by each row group's last workgroup
-        int32_t *arrivals = nullptr;
-        if (n_splits > 1) {
-            rc = ensure_arrivals(ctx, (size_t)n_groups, &arrivals);
-            if (rc != GLA_OK) return rc;
-        }
         float *out = n_splits > 1 ? part : y;
         switch (vec_pad / 16) {
         case 1:
@@ -1151,10 +1159,10 @@ int gla_matvec_q8_0(gla_ctx *ctx, const gla_q8w *w, const float *x, int n_vec, f
             return launch_splitk<4>(ctx, w, xp, xs, vec_pad, n_blocks_pad, n_vec, n_splits, out, split_stride, y, arrivals);
         }
     }
-    if (sliced) return launch_gemm<2, 1, 3>(ctx, w, xp, xs, vec_pad, n_vec, n_splits, y, part);
-    if (gemm_tiles(4, 2) >= 512) return launch_gemm<4, 2, 3>(ctx, w, xp, xs, vec_pad, n_vec, n_splits, y, nullptr);
-    if (gemm_tiles(2, 2) >= 128) return launch_gemm<2, 2, 2>(ctx, w, xp, xs, vec_pad, n_vec, n_splits, y, nullptr);
-    return launch_gemm<2, 1, 2>(ctx, w, xp, xs, vec_pad, n_vec, n_splits, y, nullptr);
+    if (sliced) return launch_gemm<2, 1, 3>(ctx, w, xp, xs, vec_pad, n_vec, n_splits, y, part, arrivals);
+    if (gemm_tiles(4, 2) >= 512) return launch_gemm<4, 2, 3>(ctx, w, xp, xs, vec_pad, n_vec, n_splits, y, nullptr, nullptr);
+    if (gemm_tiles(2, 2) >= 128) return launch_gemm<2, 2, 2>(ctx, w, xp, xs, vec_pad, n_vec, n_splits, y, nullptr, nullptr);
+    return launch_gemm<2, 1, 2>(ctx, w, xp, xs, vec_pad, n_vec, n_splits, y, nullptr, nullptr);
 }
 
 int gla_q8w_rows(const gla_q8w *w) { return w ? w->rows : -1; }

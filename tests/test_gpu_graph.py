@@ -133,3 +133,35 @@ def test_capture_that_would_grow_scratch_is_refused(backend):
         be.set_stream(None)
         s.destroy()
         w.destroy()
+
+
+@pytest.mark.parametrize("n_vec", [64, 100])
+def test_matvec_capture_after_a_longer_call(backend, n_vec):
+    """An eager projection of 400 vectors, which walks all of K, sizes the scratch for captured ones of fewer
+    vectors that take K slices; one of 100, whose own partial sums do not fit it, walks all of K. Every replay has
+    the eager call's bits."""
+    from glint_amd.attn import HipStream
+    be = backend
+    rows, cols = 6144, 2048
+    w = be.create_q8_weights(orc.q8_quantize_rows(synth.normal_rows(31, rows, cols)).reshape(-1), rows, cols)
+    x = be.buffer(synth.normal_rows(32, 400, cols))
+    y, y2 = be.empty(400 * rows * 4), be.empty(400 * rows * 4)
+    s = HipStream()
+    try:
+        be.set_stream(s)
+        be.matvec_q8_0(w, x, 400, y2)
+        be.sync()
+        g = be.capture(lambda: be.matvec_q8_0(w, x, n_vec, y))
+        for rep in range(3):
+            x.upload(synth.normal_rows(33 + rep, 400, cols))
+            g.replay()
+            be.matvec_q8_0(w, x, n_vec, y2)
+            be.sync()
+            got, want = y.download((n_vec, rows)), y2.download((n_vec, rows))
+            assert np.isfinite(want).all()
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), rep
+        g.destroy()
+    finally:
+        be.set_stream(None)
+        s.destroy()
+        w.destroy()
