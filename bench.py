@@ -837,7 +837,7 @@ def main() -> int:
         ms = t.median_ms
         tf = wl.flops_per_step() / (ms * 1e-3) / 1e12
         e_f32 = secondary["cfg4_f32"] = {
-            "workload": "Llama-3-8B causal prefill 4x2048, f32 KV cache, fp32-input MFMA",
+            "workload": "Llama-3-8B causal prefill 4x2048, f32 KV cache, fp32 (operands as two f16 pieces, three f16 MFMAs a product)",
             "value": round(tf, 2), "unit": "TFLOP/s", "ms_per_step": round(ms, 4), "timing_us": t.summary_us(),
             "frac_of_fp32_mfma_peak": round(tf / FP32_MFMA_PEAK_TFLOPS, 4),
             "frac_of_achievable_fp32_mfma": frac_of(tf, "fp32_mfma_tflops"),

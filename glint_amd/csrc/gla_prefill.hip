@@ -6,7 +6,8 @@
 // Tiling. A workgroup (4 waves) owns a block of query rows of one sequence
 // and HPW q-heads that share one KV head; every wave owns 16*NT queries of one
 // head. K/V tiles of KT=32 positions are staged in LDS once per workgroup and
-// read by all waves (GQA reuse). Per wave and tile:
+// read by all waves (GQA reuse). Per wave and tile, in the f32 body (the f16
+// pieces and bf16 take 32-wide MFMAs in the same scheme, below):
 //   S^T[key][query] = K . Q^T      v_mfma_f32_16x16x4_f32, Q^T held in VGPRs
 //   online softmax per query column (log2 domain)
 //   O^T[d][query]  += V^T . P^T    P^T is the S^T accumulator itself: the

@@ -82,7 +82,7 @@ int gla_destroy(gla_ctx *ctx);
 
 /* Run subsequent work on `hip_stream` (a hipStream_t); NULL restores the
  * context's own stream. Each stream the context has launched work on has
- * its own device scratch (decode split partials, bf16 prefill tile images,
+ * its own device scratch (decode split partials, prefill tile images,
  * matvec activation pieces), so calls queued on different streams at once
  * never share it and may overlap; calls on one stream run in order as usual.
  * That scratch is held until gla_destroy or gla_release_stream. The stream
