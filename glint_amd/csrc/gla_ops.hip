@@ -781,7 +781,16 @@ __host__ __device__ constexpr int few_stride(int nv, int kpad) {
 // per four bytes). The two block sums take the row's block scales, then the
 // four groups and the waves are summed in a fixed order. Bound: HBM on the
 // weights (34 bytes per 32).
-template <int NV>
+//
+// MFMA, for four vectors: the products run on v_mfma_f32_4x4x1 (16 blocks of 4
+// rows x 4 vectors, one element each, the same order of f32 FMAs: the same
+// bits), so a wave reads each x element from LDS once instead of once per row
+// lane: an eighth of the vector FMAs and a quarter of the LDS reads. It is faster
+// where every CU has at most one workgroup and runs there. us per call, FMAs /
+// MFMA: 4096 x 4096 8.0 / 7.5, 1024 x 4096 7.1 / 6.6, 576 x 576 and 576 x 960
+// alike, but 6144 x 4096 11.6 / 12.7, 8192 x 3584 14.6 / 18.2; three vectors
+// 4096 x 4096 7.1 / 7.6.
+template <int NV, bool MFMA>
 __global__ __launch_bounds__(kFewWaves * 64) void matvec_q8_few_kernel(const uint8_t *quants,
                                                                       const uint16_t *scales, int rows,
                                                                       int n_pairs, int cols, const float *x,
@@ -804,6 +813,13 @@ __global__ __launch_bounds__(kFewWaves * 64) void matvec_q8_few_kernel(const uin
         q = make_uint4(v.x, v.y, v.z, v.w);
         sc = *reinterpret_cast<const uint32_t *>(scales + (tp * 16 + r) * 2);  // the row's two block scales
     };
+    // MFMA: lane (r, kg) multiplies x of vector `vj`, from an LDS place
+    // swizzled so that the 16 chunks a quarter-wave reads (4 vectors x 4 groups)
+    // cover all banks, and sums the rows 4*(r/4) .. +3 of that vector
+    static_assert(!MFMA || NV == 4, "four vectors a block");
+    const int vj = lane & 3;
+    const auto swizzle = [](int v) { return MFMA ? (v & 1) * 4 + (v >> 1) * 32 : 0; };
+    const int xat = (kg * 8) ^ swizzle(vj);
     float acc[NV];
 #pragma unroll
     for (int v = 0; v < NV; v++) acc[v] = 0.0f;
@@ -813,11 +829,36 @@ __global__ __launch_bounds__(kFewWaves * 64) void matvec_q8_few_kernel(const uin
 #pragma unroll
         for (int e = 0; e < 16; e++) w[e] = (float)(int8_t)(qs[e >> 2] >> (8 * (e & 3)));
         typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+        if constexpr (MFMA) {
+            const float *xa = xl + vj * xstride + p * 64;
+            const floatx4 x0[2] = {*reinterpret_cast<const floatx4 *>(xa + xat),  // block 2p
+                                   *reinterpret_cast<const floatx4 *>(xa + (xat ^ 4))};
+            const floatx4 x1[2] = {*reinterpret_cast<const floatx4 *>(xa + (xat ^ 32)),  // block 2p + 1
+                                   *reinterpret_cast<const floatx4 *>(xa + (xat ^ 36))};
+            floatx4 t0 = {0.0f, 0.0f, 0.0f, 0.0f}, t1 = t0;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                t0 = __builtin_amdgcn_mfma_f32_4x4x1f32(w[e], x0[e >> 2][e & 3], t0, 0, 0, 0);
+                t1 = __builtin_amdgcn_mfma_f32_4x4x1f32(w[8 + e], x1[e >> 2][e & 3], t1, 0, 0, 0);
+            }
+            // the four rows' scales are the quad's: quad_perm [i i i i]
+            const uint32_t rs[4] = {(uint32_t)__builtin_amdgcn_update_dpp(0, (int)sc, 0x00, 0xf, 0xf, true),
+                                    (uint32_t)__builtin_amdgcn_update_dpp(0, (int)sc, 0x55, 0xf, 0xf, true),
+                                    (uint32_t)__builtin_amdgcn_update_dpp(0, (int)sc, 0xAA, 0xf, 0xf, true),
+                                    (uint32_t)__builtin_amdgcn_update_dpp(0, (int)sc, 0xFF, 0xf, 0xf, true)};
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const half2v s2 = __builtin_bit_cast(half2v, rs[i]);
+                acc[i] = fmaf(t0[i], (float)s2[0], acc[i]);
+                acc[i] = fmaf(t1[i], (float)s2[1], acc[i]);
+            }
+            return;
+        }
         const half2v s2 = __builtin_bit_cast(half2v, sc);
         const float s0 = (float)s2[0];
         const float s1 = (float)s2[1];
 #pragma unroll
-        for (int v = 0; v < NV; v++) {
+        for (int v = 0; v < (MFMA ? 0 : NV); v++) {
             const float *xa = xl + v * xstride + p * 64 + kg * 8;  // block 2p
             const float4 a0 = *reinterpret_cast<const float4 *>(xa);
             const float4 a1 = *reinterpret_cast<const float4 *>(xa + 4);
@@ -868,7 +909,7 @@ __global__ __launch_bounds__(kFewWaves * 64) void matvec_q8_few_kernel(const uin
 #pragma unroll
     for (int v = 0; v < NV; v++)
 #pragma unroll
-        for (int u = 0; u < kXC; u++) xl[v * xstride + threadIdx.x + u * kFewWaves * 64] = xr[v][u];  // padded row
+        for (int u = 0; u < kXC; u++) xl[v * xstride + ((threadIdx.x + u * kFewWaves * 64) ^ swizzle(v))] = xr[v][u];  // padded row
     for (int c0 = kChunk; NV == 1 && c0 < kpad; c0 += kChunk) {  // rows wider than one chunk
         float xw[NV][kXC];
 #pragma unroll
@@ -924,7 +965,7 @@ __global__ __launch_bounds__(kFewWaves * 64) void matvec_q8_few_kernel(const uin
     __syncthreads();  // x is no longer read: its LDS holds the waves' sums
     if (lane < 16) {
 #pragma unroll
-        for (int v = 0; v < NV; v++) xl[(wave * NV + v) * 16 + r] = acc[v];
+        for (int v = 0; v < NV; v++) xl[MFMA ? (wave * NV + vj) * 16 + (r & 12) + v : (wave * NV + v) * 16 + r] = acc[v];
     }
     __syncthreads();
     if ((int)threadIdx.x < NV * 16) {
@@ -944,8 +985,11 @@ int launch_few(gla_ctx *ctx, const gla_q8w *w, const float *x, float *y) {
     if (NV > 1 && kpad > few_xc(NV) * kFewWaves * 64)  // the kernel stages one chunk per vector when NV > 1
         return set_error(GLA_ERR_KERNEL, "matvec_q8_few_kernel<%d>: %d columns exceed one staging chunk", NV, kpad);
     const size_t lds = (size_t)std::max(NV * few_stride(NV, kpad), kFewWaves * NV * 16) * sizeof(float);
-    hipLaunchKernelGGL((matvec_q8_few_kernel<NV>), dim3(w->n_tiles), dim3(kFewWaves * 64), lds, ctx->stream,
-                       w->quants, w->scales, w->rows, w->n_pairs, w->cols, x, y);
+    auto kernel = matvec_q8_few_kernel<NV, false>;
+    if constexpr (NV == 4)
+        if (w->n_tiles <= ctx->n_cu) kernel = matvec_q8_few_kernel<4, true>;
+    hipLaunchKernelGGL(kernel, dim3(w->n_tiles), dim3(kFewWaves * 64), lds, ctx->stream, w->quants, w->scales, w->rows,
+                       w->n_pairs, w->cols, x, y);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "matvec_q8_few_kernel launch: %s", hipGetErrorString(e));
     return GLA_OK;

@@ -228,3 +228,16 @@ def test_matvec_q8_0_many_vectors(backend, rows, cols, n_vec):
     w = w.reshape(rows, cols)
     err = np.abs(got - x.astype(np.float64) @ w.T)
     assert np.all(err <= 2e-6 * (np.abs(x).astype(np.float64) @ np.abs(w).T) + 1e-30)
+
+
+@pytest.mark.parametrize("rows,cols", [(16, 32), (37, 96), (192, 576), (1000, 4096), (4112, 64), (8192, 96)])
+def test_matvec_q8_0_four_vectors(backend, rows, cols):
+    """Four vectors, on the matrix units up to one row tile per CU and on the vector units above: the bits of
+    one-vector calls, whose order of FMAs both keep."""
+    raw = orc.q8_quantize_rows(synth.normal_rows(911, rows, cols)).reshape(-1)
+    x = synth.normal(912, (4, cols))
+    x[1, cols // 2] = np.inf  # stays in its own vector
+    got = _matvec_gpu(backend, raw, rows, cols, x)
+    for v in range(4):
+        one = _matvec_gpu(backend, raw, rows, cols, x[v:v + 1])[0]
+        assert np.array_equal(got[v], one, equal_nan=True), v
