@@ -6,19 +6,16 @@
 // Tiling. A workgroup (4 waves) owns a block of query rows of one sequence
 // and HPW q-heads that share one KV head; every wave owns 16*NT queries of one
 // head. K/V tiles of KT=32 positions are staged in LDS once per workgroup and
-// read by all waves (GQA reuse). Per wave and tile, in the f32 body (the f16
-// pieces and bf16 take 32-wide MFMAs in the same scheme, below):
-//   S^T[key][query] = K . Q^T      v_mfma_f32_16x16x4_f32, Q^T held in VGPRs
+// read by all waves (GQA reuse). Per wave and tile:
+//   S^T[key][query] = K . Q^T      MFMA, Q^T held in VGPRs
 //   online softmax per query column (log2 domain)
-//   O^T[d][query]  += V^T . P^T    P^T is the S^T accumulator itself: the
-//                                  k-step i of a 16-key tile takes keys
-//                                  {4j + i}, j = lane / 16, which is exactly
-//                                  what accumulator register i holds.
-// Permuting the reduction index this way costs nothing and avoids any
-// register shuffle between the two products.
+//   O^T[d][query]  += V^T . P^T    P^T is packed from the lane's S^T
+//                                  accumulators: V's pieces hold the keys in
+//                                  that order, so no value changes its lane.
 #include <math.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "gla_internal.h"
 
@@ -113,7 +110,7 @@ struct SoftCap {
 };
 
 // Soft-cap and causal/window mask of one query column of a 32-key score tile
-// (sacc[mt][i]: key k0 + 16*mt + 4*lgrp + i), in place, log2 domain. The
+// (sacc[mt][i]: key kbase + 16*mt + i), in place, log2 domain. The
 // soft-cap is a template argument and the mask one wave-uniform branch per
 // tile with selects inside: written per score, both conditions became a
 // branch around every score.
@@ -143,319 +140,6 @@ __device__ __forceinline__ int window_lo(int pos, int w) {
     if (w <= 0) return 0;
     int s = pos - w + 1;
     return s > 0 ? s : 0;
-}
-
-// One tile's K/V as f32 in registers: thread u of the workgroup holds 16
-// consecutive elements (unit u / (D/16) is the key, unit % (D/16) the
-// 16-element column block) of K and of V; keys outside [klo, khi] are zero.
-template <int D, int NTHR>
-struct TileRegs {
-    static constexpr int UNITS = KT * D / 16;
-    static constexpr int PER_THREAD = (UNITS + NTHR - 1) / NTHR;
-    float4 k[PER_THREAD][4];
-    float4 v[PER_THREAD][4];
-};
-
-template <int D, int NTHR, bool Q8>
-__device__ __forceinline__ void fetch_tile(const PrefillParams &p, int b, int kvh, int k0, int klo, int khi,
-                                           TileRegs<D, NTHR> &t) {
-    const int64_t head_off = (int64_t)kvh * p.kv.head_stride;
-#pragma unroll
-    for (int j = 0; j < TileRegs<D, NTHR>::PER_THREAD; j++) {
-        const int u = threadIdx.x + j * NTHR;
-        const int key = u / (D / 16);
-        const int c16 = u - key * (D / 16);
-        const int kp = k0 + key;
-        float kf[16], vf[16];
-        if (u < TileRegs<D, NTHR>::UNITS && kp >= klo && kp <= khi) {
-            const int64_t pid = map_page(p.pm, b, kp >> 4);
-            const int slot = kp & 15;
-            if constexpr (Q8) {
-                // quants in the decode kernel's MFMA operand order (gla_internal.h)
-                const int64_t hb = pid * p.kv.page_stride + head_off;
-                const uint2 ka = *reinterpret_cast<const uint2 *>(p.kv.k + hb + q8k_off(slot, c16 * 16, D));
-                const uint2 kb = *reinterpret_cast<const uint2 *>(p.kv.k + hb + q8k_off(slot, c16 * 16 + 8, D));
-                const uint4 kq = make_uint4(ka.x, ka.y, kb.x, kb.y);
-                uint32_t vw4[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-                for (int e = 0; e < 16; e++)
-                    vw4[e >> 2] |= (uint32_t)p.kv.v[hb + q8v_off(slot, c16 * 16 + e, D)] << ((e & 3) * 8);
-                const int blk = (c16 * 16) >> 5;
-                const uint16_t *ksp = reinterpret_cast<const uint16_t *>(p.kv.ks + hb) + q8ks_off(slot, blk, D);
-                const uint16_t *vsp = reinterpret_cast<const uint16_t *>(p.kv.vs + hb) + slot * (D / 32) + blk;
-                const float ksc = __half2float(__ushort_as_half(*ksp));
-                const float vsc = __half2float(__ushort_as_half(*vsp));
-                const uint32_t kw[4] = {kq.x, kq.y, kq.z, kq.w};
-#pragma unroll
-                for (int e = 0; e < 16; e++) {  // stored quants are x + 128
-                    kf[e] = (float)((int)((kw[e >> 2] >> ((e & 3) * 8)) & 0xff) - 128) * ksc;
-                    vf[e] = (float)((int)((vw4[e >> 2] >> ((e & 3) * 8)) & 0xff) - 128) * vsc;
-                }
-            } else {
-                const int64_t base = pid * p.kv.page_stride + head_off + (int64_t)slot * p.kv.row_stride;
-                // chunk q of the lane: floats 4*c16 + q*D/4 of the row, so
-                // each load and each LDS store instruction covers whole
-                // 128-byte runs of a row (16 consecutive floats per lane
-                // made the LDS stores conflict)
-                const float4 *kp4 = reinterpret_cast<const float4 *>(p.kv.k + base) + c16;
-                const float4 *vp4 = reinterpret_cast<const float4 *>(p.kv.v + base) + c16;
-#pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    t.k[j][q] = kp4[q * (D / 16)];
-                    t.v[j][q] = vp4[q * (D / 16)];
-                }
-                continue;
-            }
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                t.k[j][q] = make_float4(kf[4 * q], kf[4 * q + 1], kf[4 * q + 2], kf[4 * q + 3]);
-                t.v[j][q] = make_float4(vf[4 * q], vf[4 * q + 1], vf[4 * q + 2], vf[4 * q + 3]);
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                t.k[j][q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                t.v[j][q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            }
-        }
-    }
-}
-
-// K and V rows in LDS: D floats + 4 of padding, so the 16 rows a 16-lane
-// group reads with 16-byte loads start in distinct bank groups.
-template <int D>
-constexpr int kRow = D + 4;
-
-template <int D, int NTHR, bool Q8>
-__device__ __forceinline__ void store_tile(const TileRegs<D, NTHR> &t, float *Ks, float *Vs) {
-#pragma unroll
-    for (int j = 0; j < TileRegs<D, NTHR>::PER_THREAD; j++) {
-        const int u = threadIdx.x + j * NTHR;
-        if (u >= TileRegs<D, NTHR>::UNITS) break;
-        const int key = u / (D / 16);
-        const int c16 = u - key * (D / 16);
-        // chunk q: floats 16*c16 + 4*q of the row (Q8) or 4*c16 + q*D/4 (f32)
-        float4 *kd = reinterpret_cast<float4 *>(Ks + key * kRow<D> + (Q8 ? c16 * 16 : c16 * 4));
-        float4 *vd = reinterpret_cast<float4 *>(Vs + key * kRow<D> + (Q8 ? c16 * 16 : c16 * 4));
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            kd[Q8 ? q : q * (D / 16)] = t.k[j][q];
-            vd[Q8 ? q : q * (D / 16)] = t.v[j][q];
-        }
-    }
-}
-
-// Workgroup: NW waves; a wave owns 16*NT queries of one q-head, the HPW
-// heads of the workgroup share one KV head (NW / HPW waves per head). K/V tiles of KT keys are
-// double-buffered in LDS: the next tile is fetched into registers while the
-// current one is multiplied, then stored to the other buffer, with one
-// barrier per tile.
-// Reduction order. Lane group g (lanes 16g..16g+15) covers the head
-// dimensions [g*D/4, (g+1)*D/4): k-step s of S^T = K.Q^T multiplies d =
-// g*D/4 + s, so a lane reads its K operands four at a time from one row.
-// O^T row R of d-tile t is d = R*DT + t, so the V^T operands a lane needs
-// for one key are DT consecutive floats, and a lane's outputs for a query
-// are the 4*DT consecutive floats [4g*DT, 4(g+1)*DT).
-template <int D>
-constexpr int kF32Lds = 4 * KT * kRow<D> * 4;  // two K and two V tiles
-
-template <int D, int NT, int NW, bool Q8, bool CAP>
-__device__ __forceinline__ void prefill_f32_body(const PrefillParams &p, uint8_t *lds, int unit, int qb0) {
-    constexpr int NTHR = NW * 64;
-    constexpr int QW = 16 * NT;  // queries per wave
-    constexpr int KS = D / 4;    // k-steps of S = K Q^T
-    constexpr int DT = D / 16;   // d tiles of O
-    float *Kb = reinterpret_cast<float *>(lds);
-    float *Vb = Kb + 2 * KT * kRow<D>;
-
-    const int n_hgrp = p.group / p.hpw;
-    const int b = unit / (p.n_kv_heads * n_hgrp);
-    const int kvh = (unit - b * p.n_kv_heads * n_hgrp) / n_hgrp;
-    const int hgrp = unit - (b * p.n_kv_heads + kvh) * n_hgrp;
-    const int waves_per_head = NW / p.hpw;
-    const int qwg = QW * waves_per_head;
-
-    const int row0 = p.q_start[b];
-    const int q_len = min(max(p.q_start[b + 1] - row0, 0), p.max_q_len);
-    const int pos0 = p.pos_offset[b];
-    if (qb0 >= q_len) return;  // qb0: first local query
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int lrow = lane & 15;
-    const int lgrp = lane >> 4;
-    const int head = kvh * p.group + hgrp * p.hpw + (wave % p.hpw);
-    const int wq0 = qb0 + (wave / p.hpw) * QW;  // first local query of this wave
-
-    // key range of the workgroup
-    const int q_last = min(q_len, qb0 + qwg) - 1;
-    const int khi = min(pos0 + q_last, p.pm.pos_limit - 1);
-    const int klo = window_lo(pos0 + qb0, p.sliding_window);
-
-    // Q^T fragments: qf[nt][s] = Q[query nt*16 + lrow][d = lgrp*KS + s]
-    float qf[NT][KS];
-#pragma unroll
-    for (int nt = 0; nt < NT; nt++) {
-        const int lq = wq0 + nt * 16 + lrow;
-        const bool ok = lq < q_len;
-        const float4 *qp = reinterpret_cast<const float4 *>(
-            p.q + ((int64_t)(row0 + (ok ? lq : 0)) * p.n_heads + head) * D + lgrp * KS);
-#pragma unroll
-        for (int s4 = 0; s4 < KS / 4; s4++) {
-            const float4 v = qp[s4];
-            qf[nt][4 * s4 + 0] = ok ? v.x * p.q_mul : 0.0f;
-            qf[nt][4 * s4 + 1] = ok ? v.y * p.q_mul : 0.0f;
-            qf[nt][4 * s4 + 2] = ok ? v.z * p.q_mul : 0.0f;
-            qf[nt][4 * s4 + 3] = ok ? v.w * p.q_mul : 0.0f;
-        }
-    }
-
-    floatx4 o[DT][NT];
-#pragma unroll
-    for (int t = 0; t < DT; t++)
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++) o[t][nt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    float m[NT], lpart[NT];
-    int qpos[NT], qlo[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; nt++) {
-        m[nt] = -INFINITY;
-        lpart[nt] = 0.0f;
-        const int lq = wq0 + nt * 16 + lrow;
-        qpos[nt] = lq < q_len ? pos0 + lq : -1;  // -1: padding query, every key masked
-        qlo[nt] = window_lo(pos0 + lq, p.sliding_window);
-    }
-
-    if (khi >= klo) {
-        const int kfirst = (klo / KT) * KT;
-        TileRegs<D, NTHR> tr;
-        fetch_tile<D, NTHR, Q8>(p, b, kvh, kfirst, klo, khi, tr);
-        store_tile<D, NTHR, Q8>(tr, Kb, Vb);
-        __syncthreads();
-        int buf = 0;
-        for (int k0 = kfirst; k0 <= khi; k0 += KT, buf ^= 1) {
-            const bool more = k0 + KT <= khi;
-            if (more) fetch_tile<D, NTHR, Q8>(p, b, kvh, k0 + KT, klo, khi, tr);
-            const float *ks = Kb + buf * KT * kRow<D>;
-            const float *vs = Vb + buf * KT * kRow<D>;
-
-            // S^T = K . Q^T
-            floatx4 sacc[2][NT];
-#pragma unroll
-            for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-                for (int nt = 0; nt < NT; nt++) sacc[mt][nt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int s4 = 0; s4 < KS / 4; s4++) {
-                float av[2][4];
-#pragma unroll
-                for (int mt = 0; mt < 2; mt++) {
-                    const float4 a = *reinterpret_cast<const float4 *>(ks + (mt * 16 + lrow) * kRow<D> + lgrp * KS +
-                                                                       4 * s4);
-                    av[mt][0] = a.x;
-                    av[mt][1] = a.y;
-                    av[mt][2] = a.z;
-                    av[mt][3] = a.w;
-                }
-                // the 2*NT accumulators in turn: a dependent MFMA every 2*NT issues
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-#pragma unroll
-                    for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-                        for (int nt = 0; nt < NT; nt++)
-                            sacc[mt][nt] =
-                                __builtin_amdgcn_mfma_f32_16x16x4f32(av[mt][e], qf[nt][4 * s4 + e], sacc[mt][nt], 0, 0, 0);
-            }
-
-            // online softmax over this tile, per query column. Only tiles that
-            // cross the diagonal, a window edge or the key range need the mask.
-            const bool interior = k0 >= klo && k0 + KT - 1 <= min(khi, pos0 + wq0) &&
-                                  (p.sliding_window <= 0 || k0 >= window_lo(pos0 + wq0 + QW - 1, p.sliding_window));
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++) {
-                floatx4 col[2] = {sacc[0][nt], sacc[1][nt]};
-                cap_and_mask<CAP>(col, p.softcap, interior, k0 + 4 * lgrp, qpos[nt], qlo[nt], klo, khi);
-                sacc[0][nt] = col[0];
-                sacc[1][nt] = col[1];
-                float mx = -INFINITY;
-#pragma unroll
-                for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) mx = fmaxf(mx, sacc[mt][nt][i]);
-                mx = max_rows4(mx);
-                const float m_new = fmaxf(m[nt], mx);
-                if (m_new == -INFINITY) {
-#pragma unroll
-                    for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-                        for (int i = 0; i < 4; i++) sacc[mt][nt][i] = 0.0f;
-                    continue;
-                }
-                const float rs = fast_exp2(m[nt] - m_new);
-                m[nt] = m_new;
-                float ls = 0.0f;
-#pragma unroll
-                for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const float pv = fast_exp2(sacc[mt][nt][i] - m_new);
-                        sacc[mt][nt][i] = pv;
-                        ls += pv;
-                    }
-                lpart[nt] = lpart[nt] * rs + ls;
-                if (__ballot(rs != 1.0f)) {  // the running max moved for some query
-#pragma unroll
-                    for (int t = 0; t < DT; t++) o[t][nt] *= rs;
-                }
-            }
-
-            // O^T += V^T . P^T
-#pragma unroll
-            for (int mt = 0; mt < 2; mt++) {
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float *vrow = vs + (mt * 16 + 4 * lgrp + i) * kRow<D> + lrow * DT;
-                    float av[DT];
-#pragma unroll
-                    for (int t4 = 0; t4 < DT / 4; t4++) {
-                        const float4 a = reinterpret_cast<const float4 *>(vrow)[t4];
-                        av[4 * t4] = a.x;
-                        av[4 * t4 + 1] = a.y;
-                        av[4 * t4 + 2] = a.z;
-                        av[4 * t4 + 3] = a.w;
-                    }
-#pragma unroll
-                    for (int t = 0; t < DT; t++)
-#pragma unroll
-                        for (int nt = 0; nt < NT; nt++)
-                            o[t][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[t], sacc[mt][nt][i], o[t][nt], 0, 0, 0);
-                }
-            }
-
-            if (more) store_tile<D, NTHR, Q8>(tr, Kb + (buf ^ 1) * KT * kRow<D>, Vb + (buf ^ 1) * KT * kRow<D>);
-            __syncthreads();
-        }
-    }
-
-    // normalise and store: lane holds O^T[d = (4*lgrp + r)*DT + t][query lrow]
-#pragma unroll
-    for (int nt = 0; nt < NT; nt++) {
-        float lt = lpart[nt];
-        lt = sum_rows4(lt);
-        const int lq = wq0 + nt * 16 + lrow;
-        if (lq >= q_len) continue;
-        const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
-        float *op = p.out + ((int64_t)(row0 + lq) * p.n_heads + head) * D + 4 * lgrp * DT;
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-#pragma unroll
-            for (int t4 = 0; t4 < DT / 4; t4++)
-                *reinterpret_cast<float4 *>(op + r * DT + 4 * t4) =
-                    make_float4(o[4 * t4][nt][r] * inv, o[4 * t4 + 1][nt][r] * inv, o[4 * t4 + 2][nt][r] * inv,
-                                o[4 * t4 + 3][nt][r] * inv);
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -930,6 +614,20 @@ __device__ __forceinline__ void lds_copy16(const uint8_t *sbase, uint32_t voff, 
         : "memory");
 }
 
+// 4 bytes per lane from sbase + voff into LDS at m0 + 4 * lane.
+__device__ __forceinline__ void lds_copy4(const uint8_t *sbase, uint32_t voff, uint32_t m0) {
+    uint32_t save;
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %3\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dword %1, %2\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(save)
+        : "v"(voff), "s"(sbase), "s"(m0)
+        : "memory");
+}
+
 template <int N>
 __device__ __forceinline__ void wait_vm() {
     static_assert(N >= 0 && N < 64, "vmcnt range");
@@ -1161,70 +859,169 @@ __global__ __launch_bounds__(kBf16sWaves<D> * 64, kBf16sOccupancy<D>) void prefi
 
 // ---------------------------------------------------------------------------
 // fp32 prefill on the f16 matrix cores. Every f32 operand is two f16 pieces
-// (hi = f16(x), lo = f16(x - hi): 22 bits) after a power-of-two scaling, and a
-// product is three MFMAs, hi.hi + hi.lo + lo.hi; the dropped lo.lo is 2^-24 of
-// the product. Products of f16 pieces are exact in the f32 accumulators, and a
-// 32-wide MFMA rounds once where the 4-wide f32 one rounds eight times, so the
-// error against 64 bits does not grow: 4 prompts of 2,048 at 32/8 heads, d =
-// 128, have a relative error of 2.7e-7 (f32 MFMAs: 4.4e-7). Three f16 MFMAs do
+// after a power-of-two scaling, hi = f16(x) and lo = f16((x - hi) * 2^11): 22
+// bits of x wherever hi is a normal f16, which is 29 binades below 2^15. A
+// product is three MFMAs, hi.hi and, 2^-11 below, hi.lo + lo.hi; the dropped
+// lo.lo is 2^-24 of it. Products of f16 pieces are exact in the f32
+// accumulators, and a 32-wide MFMA rounds once where the 4-wide f32 one rounds
+// eight times, so the error against 64 bits is smaller: 4 prompts of 2,048 at
+// 32/8 heads, d = 128, 2.0e-7 relative (f32 MFMAs: 4.4e-7). Three f16 MFMAs do
 // the work of a 16x16x32 tile in 48 cycles, the f32 ones in 256: the same four
-// prompts take 375 us, of them 23 the staging (f32 MFMAs: 1,083 us), 367
-// TFLOP/s. What bounds it is the chain S -> softmax -> O at two waves per SIMD:
-// a tile takes a workgroup 2.2 us and its MFMAs 0.65 us of each wave's SIMD.
+// prompts take 394 us, of them 23 the staging (f32 MFMAs: 1,083 us). What bounds
+// it is the chain S -> softmax -> O at two waves per SIMD: matrix and vector
+// cycles add up.
 //
-// Scaling. K takes one power of two per 32-key tile, undone on the scores (with
-// the query's own); V one per tile as well, which is the unit O is accumulated
-// in: when it changes, O is moved to the new unit (an exact product). The
-// exponents are rounded up to multiples of 4, so tiles of like magnitude share
-// a unit. p = 2^(s - m) is held below 2^14 (kSplitP).
+// Scaling. A row's result follows from the row and the keys it attends alone,
+// bit for bit, whatever rows, chunks and sequences share its call: every scale
+// belongs to one key or to one row. A key's K and V each take a power of two
+// from their own largest value, one for eight binades (kClass), and a query row
+// one from its own. K's and the query's are undone on the scores. V's is carried
+// by the probability: O accumulates p * 2^(E - R) times the scaled V, E the key's
+// exponent and R the row's: the largest E it has attended, moved (with O) when
+// one passes it by more than 2^2. So the products' operand is largest where the
+// contribution p * V is, and it is the small contributions that reach the end of
+// f16's range. Where all keys that a workgroup attends share their exponents and
+// nothing is odd, as with most data, its loop over the tiles holds the scales as
+// constants (`plain`); otherwise it takes them key by key. Both give the same bits.
 //
-// What the pieces cannot carry at f32 precision goes through the f32 body
-// above, decided per workgroup: a tile that holds an infinity or a NaN, whose
-// largest value lies outside [2^-45, 2^45] (K) or [2^-20, 2^20] (V), or whose
-// values differ too much in magnitude (kSplitRange), and a query row with a
-// non-finite value or a maximum outside [2^-45, 2^45]. A value x of a tile whose
-// largest is M has an error of at most max(2^-23 |x|, 2^-35 M).
+// What the pieces cannot hold is named per key ("odd"): infinities and NaN, K
+// with a run of 8 dims below 2^-20 of its largest value, V's values below kSmall
+// (scaled). The scores of an odd key, or of a query row that is odd in the same
+// way, come from the f32 MFMA; odd V values are zero in the image, and their
+// products are added in f32 for the rows that attend them.
 typedef _Float16 half8p __attribute__((ext_vector_type(8)));
 
-constexpr int kSplitP = 6;            // p is scaled by 2^6: with the lazy maximum's 2^8 it stays below 2^14
-// How much smaller than a tile's largest value that of 8 dims of a key (K) or
-// of 8 keys of a dim (V) may be: 2^12; in a tile that is not full 2^20, since
-// there a V run may hold one key, whose value is small by chance.
-constexpr float kSplitRange = 0x1p12f, kSplitRangePart = 0x1p20f;
+constexpr float kMLowest = -3.402823466e38f;  // a row's maximum before its first key
+constexpr float kLazyF32 = 4.0f;  // the lazy maximum's margin: p = 2^(s - m) stays below 2^4, whatever m's ulp
+constexpr int kLazyExp = 2;       // R's: p * 2^(E - R) stays below 2^6
+constexpr int kScaleP = 9;        // and in f16 below 2^15
+constexpr int kTop = 15;          // scaled K, V and q stay below 2^15
+constexpr int kNoExp = -300;      // R before a row's first key
+constexpr float kSmall = 0x1p-16f;  // scaled V values below it are odd
 
 // A tile's image: K hi, K lo, V hi, V lo, each 64*D bytes in the piece order
 // of the bf16 image.
 template <int D>
 constexpr int kSplitImage = 256 * D;
-// What the attention needs to know of a tile: the factor that undoes K's
-// scale (NaN: the tile takes the f32 body), and V's scale (0: V is all zero).
-struct TileMeta {
-    float k_inv, v_scale;
+// What the attention needs to know of a tile.
+struct TileHead {
+    int32_t exps;           // the keys' exponents (key_exps); kMixed: they differ
+    uint32_t odd_k, odd_v;  // odd keys, a bit each
 };
+struct TileMeta {
+    TileHead head;
+    int32_t exps[KT];  // by key, where it is in range
+    uint32_t pad[29];  // 256 bytes: four for each lane of a wave
+};
+static_assert(sizeof(TileMeta) == 256, "one 4-byte copy per lane");
+constexpr int32_t kMixed = -1;
+// The exponents of a key's K and V in one number.
+__device__ __forceinline__ int32_t key_exps(int k, int v) { return (k + 1024) << 12 | (v + 1024); }
+__device__ __forceinline__ int k_exp_of(int32_t exps) { return (exps >> 12) - 1024; }
+__device__ __forceinline__ int v_exp_of(int32_t exps) { return (exps & 0xfff) - 1024; }
 
+// The pieces of 8 values times mul.
 __device__ __forceinline__ void split8(const float (&x)[8], float mul, half8p &hi, half8p &lo) {
 #pragma unroll
     for (int j = 0; j < 8; j++) {
         const float t = x[j] * mul;
         const _Float16 h = (_Float16)t;
         hi[j] = h;
-        lo[j] = (_Float16)(t - (float)h);
+        lo[j] = (_Float16)fmaf((float)h, -2048.0f, t * 2048.0f);
     }
 }
 
-// 2^(14 - e) for the exponent e of m (m in [2^(e-1), 2^e)), e rounded up to a
-// multiple of STEP: m times it lies in [2^(14-STEP), 2^14).
-template <int STEP>
-__device__ __forceinline__ int split_exponent(float m) {
-    int e = (int)((__float_as_uint(m) >> 23) & 0xff) - 126;
-    e = (e + STEP - 1) & ~(STEP - 1);
-    return 14 - e;
+// The exponent e of a positive value m, from its bits: m is in [2^(e-1), 2^e). At
+// least -100 (smaller values keep fewer bits).
+__device__ __forceinline__ int exponent_of(uint32_t bits) { return max((int)(bits >> 23) - 126, -100); }
+// A key's: e rounded up to 5 more than a multiple of 8, so that the largest
+// values of [1/8, 32) share one. (A key of zeros has that of 1.)
+constexpr int kClass = 8;
+__device__ __forceinline__ int class_of(uint32_t bits) {
+    return bits ? (exponent_of(bits) + kClass * 16 - 6 + kClass) / kClass * kClass - kClass * 16 + 5 : 5;
 }
 __device__ __forceinline__ float pow2f(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
 
+// max of |x| over 8 values, as bits (an infinity or a NaN is the largest)
+__device__ __forceinline__ uint32_t top_bits(const float (&x)[8]) {
+    uint32_t t = 0;
+#pragma unroll
+    for (int j = 0; j < 8; j++) t = max(t, __float_as_uint(x[j]) & 0x7fffffffu);
+    return t;
+}
+constexpr uint32_t kInfBits = 0x7f800000u;
+// Whether a run of 8 values, the largest `run`, is too small beside `top`.
+__device__ __forceinline__ bool run_is_odd(uint32_t run, uint32_t top) { return run != 0 && run + (20u << 23) < top; }
+
+// max over the lanes that share lane % N (N = 2, 4 or 8)
+template <int N>
+__device__ __forceinline__ uint32_t umax_stride(uint32_t x) {
+    if constexpr (N <= 2) x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, x, 0x122, 0xf, 0xf, true));  // row_ror 2, 4, 8
+    if constexpr (N <= 4) x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, x, 0x124, 0xf, 0xf, true));
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, x, 0x128, 0xf, 0xf, true));
+    return umax_rows4(x);
+}
+// max over N neighbouring lanes (N = 8, 16 or 32)
+template <int N>
+__device__ __forceinline__ uint32_t umax_group(uint32_t x) {
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, x, 0xB1, 0xf, 0xf, true));   // quad_perm [1 0 3 2]
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, x, 0x4E, 0xf, 0xf, true));   // quad_perm [2 3 0 1]
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, x, 0x141, 0xf, 0xf, true));  // row_half_mirror
+    if constexpr (N >= 16) x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, x, 0x128, 0xf, 0xf, true));  // row_ror 8
+    if constexpr (N >= 32) {
+        const auto a = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        x = max(a[0], a[1]);
+    }
+    return x;
+}
+
+// One element of a cached K row (page and head offset in hb).
+template <int D, bool Q8>
+__device__ __forceinline__ float k_element(const PrefillParams &p, int64_t hb, int slot, int d) {
+    if constexpr (Q8) {
+        const uint16_t sc = reinterpret_cast<const uint16_t *>(p.kv.ks + hb)[q8ks_off(slot, d >> 5, D)];
+        return (float)((int)p.kv.k[hb + q8k_off(slot, d, D)] - 128) * __half2float(__ushort_as_half(sc));
+    } else {
+        return reinterpret_cast<const float *>(p.kv.k + hb + (int64_t)slot * p.kv.row_stride)[d];
+    }
+}
+
+// V of a cached row at the dims 16*t + 4*lgrp + r that a lane's O holds. (The
+// addresses are opaque so that nothing of them is kept in registers over the
+// tiles that need none.)
+template <int D, bool Q8>
+struct LaneV {
+    const uint8_t *v;
+    const uint16_t *scale;
+    __device__ __forceinline__ LaneV(const PrefillParams &p, int64_t hb, int slot, int lgrp) {
+        if constexpr (Q8) {
+            v = p.kv.v + hb + q8v_off(slot, 4 * lgrp, D);
+            scale = reinterpret_cast<const uint16_t *>(p.kv.vs + hb) + slot * (D / 32);
+            asm volatile("" : "+v"(scale));
+        } else {
+            v = p.kv.v + hb + (int64_t)slot * p.kv.row_stride + 16 * lgrp;
+            scale = nullptr;
+        }
+        asm volatile("" : "+v"(v));
+    }
+    __device__ __forceinline__ float operator()(int t, int r) const {
+        if constexpr (Q8) {
+            return (float)((int)v[(t >> 2) * 1024 + r * 16 + (t & 3) * 4] - 128) * __half2float(__ushort_as_half(scale[t >> 1]));
+        } else {
+            return reinterpret_cast<const float *>(v)[16 * t + r];
+        }
+    }
+};
+
+// Whether the image holds V value v of a key with scale 2^(kTop - e) as zero.
+__device__ __forceinline__ bool v_is_odd(float v, float scale) {
+    const float t = fabsf(v) * scale;
+    return !(t < INFINITY) || (t < kSmall && t > 0.0f);
+}
+
 // One 32-key tile of a (sequence, KV head) pair on its way from the cache to
 // its pieces, by 256 threads: fetch() issues the loads, convert() finds the
-// tile's scales and hands out the pieces.
+// keys' exponents and hands out the pieces.
 // K piece i is 8 consecutive dims of one key, V piece i 8 keys of one dim.
 template <int D>
 __device__ __forceinline__ int k_piece_key(int i) { return i / (D / 8 * 16) * 16 + (i & 15); }
@@ -1233,23 +1030,31 @@ __device__ __forceinline__ int k_piece_dim(int i) { return (i % (D / 8 * 16) >> 
 __device__ __forceinline__ int v_piece_key(int i, int j) { return (j >> 2) * 16 + 4 * ((i >> 4) & 3) + (j & 3); }
 __device__ __forceinline__ int v_piece_dim(int i) { return 16 * (i >> 6) + (i & 15); }
 
-// What convert() needs in LDS.
+// What convert() needs in LDS; odd[] is zero between tiles.
 template <int D, bool Q8>
 struct SplitAux {
-    uint4 ext[4];  // per wave, as bits: largest |K|, smallest non-zero run maximum of K; the same of V
-    TileMeta meta;
+    int k_exp[KT], v_exp[KT];
+    uint32_t odd[2];
     uint32_t pad[2];
-    float v[Q8 ? 1 : KT][Q8 ? 4 : D + 4];  // f32 rows of V, read back along the keys
+    TileMeta meta;
+    float v[Q8 ? 1 : KT][Q8 ? 4 : D + 4];  // scaled rows of V, read back along the keys
 };
 
 template <int D, bool Q8>
 struct SplitTile {
     static constexpr int NK = 4 * D / 256;  // 16-byte pieces of K (and of V) per thread
+    static constexpr int KPW = 512 / D;     // f32: whole K rows per wave and round, the low bits of the lane
     // f32: the rows' own 16-byte loads; Q8_0: quants and scales
     floatx4 ka[Q8 ? 1 : NK][2], va[Q8 ? 1 : NK][2];
     uint2 kw[Q8 ? NK : 1];
     uint32_t vw[Q8 ? NK : 1][2];
     uint16_t ks[Q8 ? NK : 1], vs[Q8 ? NK : 1][8];
+    uint16_t row_scale[Q8 ? D / 32 : 1];  // threads 0..63: all scales of one key's K (0..31) or V
+
+    static __device__ __forceinline__ int k_row(int r) {  // f32: the key of the thread's piece r
+        return ((int)(threadIdx.x >> 6) + 4 * r) * KPW + (int)(threadIdx.x & (KPW - 1));
+    }
+    static __device__ __forceinline__ int k_col(int) { return (int)(threadIdx.x & 63) / KPW; }  // its dims / 8
 
     // keys outside [klo, khi] are zero (khi >= 0, and the tile meets the range)
     __device__ __forceinline__ void fetch(const PrefillParams &p, int b, int kvh, int k0, int klo, int khi) {
@@ -1257,6 +1062,15 @@ struct SplitTile {
         const int64_t hb0 = map_page(p.pm, b, min(k0, khi) >> 4) * p.kv.page_stride + head_off;
         const int64_t hb1 = map_page(p.pm, b, min(k0 + 16, khi) >> 4) * p.kv.page_stride + head_off;
         if constexpr (Q8) {
+            if (threadIdx.x < 64) {
+                const int key = threadIdx.x & 31;
+                const int64_t hb = key < 16 ? hb0 : hb1;
+#pragma unroll
+                for (int blk = 0; blk < D / 32; blk++)
+                    row_scale[blk] = threadIdx.x < 32
+                                         ? reinterpret_cast<const uint16_t *>(p.kv.ks + hb)[q8ks_off(key & 15, blk, D)]
+                                         : reinterpret_cast<const uint16_t *>(p.kv.vs + hb)[(key & 15) * (D / 32) + blk];
+            }
 #pragma unroll
             for (int r = 0; r < NK; r++) {
                 const int i = threadIdx.x + 256 * r;
@@ -1292,14 +1106,13 @@ struct SplitTile {
             }
 #pragma unroll
             for (int r = 0; r < NK; r++) {
-                const int i = threadIdx.x + 256 * r;
-                const int key = k_piece_key<D>(i);
+                const int key = k_row(r);
                 const int kp = k0 + key;
                 ka[r][0] = ka[r][1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
                 if (kp >= klo && kp <= khi) {
                     const float *kr = reinterpret_cast<const float *>(p.kv.k + (key < 16 ? hb0 : hb1) +
                                                                       (int64_t)(kp & 15) * p.kv.row_stride) +
-                                      k_piece_dim<D>(i);
+                                      8 * k_col(r);
                     ka[r][0] = *reinterpret_cast<const floatx4 *>(kr);
                     ka[r][1] = *reinterpret_cast<const floatx4 *>(kr + 4);
                 }
@@ -1328,85 +1141,130 @@ struct SplitTile {
         }
     }
 
-    // put(i, k_hi, k_lo, v_hi, v_lo) takes piece i of each image, unless the
-    // pieces cannot carry the tile (aux.meta.k_inv is NaN). No thread may
-    // still be reading aux; after the next barrier aux.meta may be read.
-    template <typename Put>
-    __device__ __forceinline__ void convert(SplitAux<D, Q8> &aux, int k0, int klo, int khi, Put put) const {
-        float kf[NK][8], vf[NK][8];
-        if constexpr (!Q8) {
+    // put_k(i, hi, lo) and put_v(i, hi, lo) take piece i of each image. No
+    // thread may still be reading aux; after the next barrier aux.meta may be read.
+    template <typename PutK, typename PutV>
+    __device__ __forceinline__ void convert(SplitAux<D, Q8> &aux, int k0, int klo, int khi, PutK put_k, PutV put_v) const {
+        half8p hi, lo;
+        if constexpr (Q8) {
+            // exponents from a key's scales: a value is at most 128 of them,
+            // at least 1 where it is not zero
+            if (threadIdx.x < 64) {
+                const int key = threadIdx.x & 31;
+                const int kp = k0 + key;
+                uint32_t top = 0, low = 0xffffffffu;
+                bool bad = false;
+#pragma unroll
+                for (int blk = 0; blk < D / 32; blk++) {
+                    const float x = fabsf(__half2float(__ushort_as_half(row_scale[blk])));
+                    const uint32_t bits = __float_as_uint(x);
+                    const bool finite = bits < kInfBits;
+                    bad = bad || !finite;
+                    if (finite && bits) {
+                        top = max(top, bits);
+                        low = min(low, bits);
+                    }
+                }
+                const bool in = kp >= klo && kp <= khi;
+                const int e = class_of(in && top ? top + (7u << 23) : 0);
+                const bool small = top && (threadIdx.x < 32 ? low + (13u << 23) < top
+                                                            : __uint_as_float(low) * pow2f(kTop - e) < kSmall);
+                (threadIdx.x < 32 ? aux.k_exp : aux.v_exp)[key] = e;
+                if (in && (bad || small)) atomicOr(&aux.odd[threadIdx.x >> 5], 1u << key);
+            }
+            float kf[NK][8], vf[NK][8];
+            dequantize(k0, klo, khi, kf, vf);
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < NK; r++) {
+                const int i = threadIdx.x + 256 * r;
+                split8(kf[r], pow2f(kTop - aux.k_exp[k_piece_key<D>(i)]), hi, lo);
+                put_k(i, hi, lo);
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const float sc = pow2f(kTop - aux.v_exp[v_piece_key(i, j)]);
+                    if (aux.odd[1] && v_is_odd(vf[r][j], sc)) vf[r][j] = 0.0f;
+                    vf[r][j] *= sc;
+                }
+                split8(vf[r], 1.0f, hi, lo);
+                put_v(i, hi, lo);
+            }
+        } else {
 #pragma unroll
             for (int r = 0; r < NK; r++) {
                 const int u = threadIdx.x + 256 * r;
                 const int key = u / (D / 8);
-                floatx4 *dst = reinterpret_cast<floatx4 *>(&aux.v[key][8 * (u - key * (D / 8))]);
-                dst[0] = va[r][0];
-                dst[1] = va[r][1];
+                float x[8];
+                uint32_t low = 0xffffffffu;  // of the non-zero values' bits, less 1
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    x[j] = va[r][j >> 2][j & 3];
+                    low = min(low, (__float_as_uint(x[j]) & 0x7fffffffu) - 1u);
+                }
+                uint32_t top = umax_group<D / 8>(top_bits(x));
+                if (__ballot(top >= kInfBits)) {  // of the finite values
+                    top = 0;
+#pragma unroll
+                    for (int j = 0; j < 8; j++) {
+                        const uint32_t bits = __float_as_uint(x[j]) & 0x7fffffffu;
+                        top = max(top, bits < kInfBits ? bits : 0);
+                    }
+                    top = umax_group<D / 8>(top);
+                }
+                const int e = class_of(top);
+                const float sc = pow2f(kTop - e);
+                if (top_bits(x) > top || __uint_as_float(low + 1u) * sc < kSmall) {
+#pragma unroll
+                    for (int j = 0; j < 8; j++) x[j] = v_is_odd(x[j], sc) ? 0.0f : x[j];
+                    if (low != 0xffffffffu) atomicOr(&aux.odd[1], 1u << key);
+                }
+#pragma unroll
+                for (int j = 0; j < 8; j++) x[j] *= sc;
+                const int c = u - key * (D / 8);
+                if (c == 0) aux.v_exp[key] = e;
+                floatx4 *dst = reinterpret_cast<floatx4 *>(&aux.v[key][8 * c]);
+                dst[0] = floatx4{x[0], x[1], x[2], x[3]};
+                dst[1] = floatx4{x[4], x[5], x[6], x[7]};
+            }
+#pragma unroll
+            for (int r = 0; r < NK; r++) {
+                const int key = k_row(r), c = k_col(r);
+                float x[8];
+#pragma unroll
+                for (int j = 0; j < 8; j++) x[j] = ka[r][j >> 2][j & 3];
+                const uint32_t run = top_bits(x);
+                const uint32_t top = umax_stride<KPW>(run);
+                const int e = class_of(top < kInfBits ? top : 0);
+                if (top >= kInfBits || run_is_odd(run, top)) atomicOr(&aux.odd[0], 1u << key);
+                if (c == 0) aux.k_exp[key] = e;
+                split8(x, pow2f(kTop - e), hi, lo);
+                put_k(((key >> 4) * (D / 8) + c) * 16 + (key & 15), hi, lo);
             }
             __syncthreads();
-        }
-        if constexpr (Q8) {
-            dequantize(k0, klo, khi, kf, vf);
-        } else {
 #pragma unroll
             for (int r = 0; r < NK; r++) {
                 const int i = threadIdx.x + 256 * r;
+                float x[8];
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    kf[r][j] = ka[r][j >> 2][j & 3];
-                    vf[r][j] = aux.v[v_piece_key(i, j)][v_piece_dim(i)];
-                }
+                for (int j = 0; j < 8; j++) x[j] = aux.v[v_piece_key(i, j)][v_piece_dim(i)];
+                split8(x, 1.0f, hi, lo);
+                put_v(i, hi, lo);
             }
         }
-        // magnitudes, as the bits of |x| (an infinity or a NaN is the largest)
-        uint32_t ktop = 0, klow = 0xffffffffu, vtop = 0, vlow = 0xffffffffu;
-#pragma unroll
-        for (int r = 0; r < NK; r++) {
-            uint32_t km = 0, vm = 0;
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                km = max(km, __float_as_uint(kf[r][j]) & 0x7fffffffu);
-                vm = max(vm, __float_as_uint(vf[r][j]) & 0x7fffffffu);
+        if (threadIdx.x < 64) {
+            const int key = threadIdx.x & 31;
+            const int32_t exps = key_exps(aux.k_exp[key], aux.v_exp[key]);
+            const uint32_t odd_k = aux.odd[0], odd_v = aux.odd[1];
+            const int kp = k0 + key;
+            const bool in = kp >= klo && kp <= khi;
+            const uint32_t keys = (uint32_t)__ballot(in);
+            const int32_t first = __builtin_amdgcn_readlane(exps, __builtin_ctz(keys));  // (a tile has a key in range)
+            const bool same = !__ballot(in && exps != first);
+            if (threadIdx.x < 32) aux.meta.exps[key] = exps;
+            if (threadIdx.x == 0) {
+                aux.meta.head = TileHead{same ? first : kMixed, odd_k, odd_v};
+                aux.odd[0] = aux.odd[1] = 0;
             }
-            ktop = max(ktop, km);
-            klow = min(klow, km ? km : 0xffffffffu);
-            vtop = max(vtop, vm);
-            vlow = min(vlow, vm ? vm : 0xffffffffu);
-        }
-        const uint4 mine = make_uint4(wave_extreme<true>(ktop), wave_extreme<false>(klow), wave_extreme<true>(vtop),
-                                      wave_extreme<false>(vlow));
-        if ((threadIdx.x & 63) == 0) aux.ext[threadIdx.x >> 6] = mine;
-        __syncthreads();
-#pragma unroll
-        for (int w = 0; w < 4; w++) {
-            const uint4 x = aux.ext[w];
-            ktop = max(w ? ktop : 0, x.x);
-            klow = min(w ? klow : 0xffffffffu, x.y);
-            vtop = max(w ? vtop : 0, x.z);
-            vlow = min(w ? vlow : 0xffffffffu, x.w);
-        }
-        const float kmax = __uint_as_float(ktop), vmax = __uint_as_float(vtop);
-        const float range = k0 >= klo && k0 + KT - 1 <= khi ? kSplitRange : kSplitRangePart;
-        bool plain = ktop < 0x7f800000u && vtop < 0x7f800000u;
-        int ke = 0, ve = 0;
-        if (plain && ktop) {
-            plain = kmax >= 0x1p-45f && kmax <= 0x1p45f && __uint_as_float(klow) * range >= kmax;
-            ke = split_exponent<4>(kmax);
-        }
-        if (plain && vtop) {
-            plain = vmax >= 0x1p-20f && vmax <= 0x1p20f && __uint_as_float(vlow) * range >= vmax;
-            ve = split_exponent<4>(vmax);
-        }
-        if (threadIdx.x == 0)
-            aux.meta = TileMeta{plain ? pow2f(-ke) : __uint_as_float(0x7fc00000u), vtop ? pow2f(ve) : 0.0f};
-        if (!plain) return;
-        const float kmul = pow2f(ke), vmul = pow2f(ve);
-#pragma unroll
-        for (int r = 0; r < NK; r++) {
-            half8p kh, kl, vh, vl;
-            split8(kf[r], kmul, kh, kl);
-            split8(vf[r], vmul, vh, vl);
-            put(threadIdx.x + 256 * r, kh, kl, vh, vl);
         }
     }
 };
@@ -1431,15 +1289,21 @@ __global__ __launch_bounds__(256) void stage_split_kernel(const PrefillParams p,
     __shared__ __attribute__((aligned(16))) SplitAux<D, Q8> aux;
     SplitTile<D, Q8> tile;
     tile.fetch(p, b, kvh, k0, klo, khi);
+    if (threadIdx.x < 2) aux.odd[threadIdx.x] = 0;
+    __syncthreads();
     const int64_t at = (int64_t)blockIdx.y * n_tiles + t;
     uint8_t *dst = img + at * kSplitImage<D>;
-    tile.convert(aux, k0, klo, khi, [&](int i, const half8p &kh, const half8p &kl, const half8p &vh, const half8p &vl) {
-        *reinterpret_cast<half8p *>(dst + (int64_t)i * 16) = kh;
-        *reinterpret_cast<half8p *>(dst + 64 * D + (int64_t)i * 16) = kl;
-        *reinterpret_cast<half8p *>(dst + 128 * D + (int64_t)i * 16) = vh;
-        *reinterpret_cast<half8p *>(dst + 192 * D + (int64_t)i * 16) = vl;
-    });
-    if (threadIdx.x == 0) meta[at] = aux.meta;
+    const auto put = [&](uint8_t *to) {
+        return [to](int i, const half8p &hi, const half8p &lo) {
+            *reinterpret_cast<half8p *>(to + i * 16) = hi;
+            *reinterpret_cast<half8p *>(to + 64 * D + i * 16) = lo;
+        };
+    };
+    tile.convert(aux, k0, klo, khi, put(dst), put(dst + 128 * D));
+    __syncthreads();
+    constexpr int WORDS = sizeof(TileMeta) / 4;
+    if (threadIdx.x < WORDS)
+        reinterpret_cast<uint32_t *>(meta + at)[threadIdx.x] = reinterpret_cast<const uint32_t *>(&aux.meta)[threadIdx.x];
 }
 
 // The staging launch of the bf16 path.
@@ -1552,15 +1416,14 @@ __global__ __launch_bounds__(256) void stage_bf16_kernel(const PrefillParams p, 
 }
 
 // Waves per SIMD the kernel's registers are sized for; LDS holds two tiles of
-// a workgroup (or the f32 body's buffers): d = 64 35 KB, d = 128 68 KB,
-// d = 256 133 KB. A workgroup that converts its own tiles holds one image and
-// the conversion's buffers, and the next tile's loads in registers (not at
-// d = 256, whose registers are full).
-template <int D, bool STAGED>
-constexpr int kSplitOccupancy = !STAGED ? (D == 64 ? 2 : 1) : (D == 64 ? 3 : (D == 128 ? 2 : 1));
+// a workgroup: d = 64 32 KB, d = 128 64 KB, d = 256 128 KB. A workgroup that
+// converts its own tiles holds one image and the conversion's buffers, and the
+// next tile's loads in registers (not at d = 256, whose registers are full).
+template <int D, bool STAGED, int NT>
+constexpr int kSplitOccupancy = !STAGED ? (D == 64 ? 2 : 1) : (D == 64 ? 4 - NT : (D == 128 ? 2 : 1));
 
 template <int D, bool Q8, bool CAP, bool STAGED, int NT>
-__global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED>)) void prefill_split_kernel(const PrefillParams p,
+__global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill_split_kernel(const PrefillParams p,
                                                                                 const uint8_t *img,
                                                                                 const TileMeta *meta, int n_tiles,
                                                                                 int pair0) {
@@ -1571,7 +1434,9 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED>)) void prefill_spl
     constexpr int IMG = kSplitImage<D>;
     constexpr int CPW = IMG / 1024 / NW;  // kilobyte copies per wave and tile
     constexpr int AUX = IMG + (int)sizeof(SplitAux<D, Q8>);
-    constexpr int LDS = std::max(kF32Lds<D>, STAGED ? 2 * IMG : AUX);
+    constexpr int SROW = D + 4;  // an output row in LDS
+    constexpr int METAS = 2 * IMG;  // staged: where the two tiles' TileMeta are
+    constexpr int LDS = std::max(STAGED ? METAS + 2 * (int)sizeof(TileMeta) : AUX, NW * 16 * SROW * 4);
     __shared__ __attribute__((aligned(16))) uint8_t lds[LDS];
 
     const int n_hgrp = p.group / p.hpw;
@@ -1613,26 +1478,45 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED>)) void prefill_spl
 #pragma unroll
         for (int c = 0; c < CPW; c++) {
             const int piece = wave * CPW + c;
-            lds_copy16(src, (uint32_t)(piece * 1024 + lane * 16), dst + piece * 1024);
+            lds_copy16(src + piece * 1024, (uint32_t)(lane * 16), dst + piece * 1024);
         }
     };
 
+    const auto issue_meta = [&](int i) __attribute__((always_inline)) {
+        if (wave == 0)
+            lds_copy4(reinterpret_cast<const uint8_t *>(unit_meta + i), (uint32_t)(lane * 4),
+                      ring + METAS + (uint32_t)((i & 1) * sizeof(TileMeta)));
+    };
+
     if (STAGED && n > 0) issue(0);
-    // tiles and queries that the pieces cannot carry
-    bool odd = false;
-    for (int i = tid; STAGED && i < n; i += 256) odd = odd || unit_meta[i].k_inv != unit_meta[i].k_inv;
+    // whether the tiles' keys share their exponents and none is odd
+    bool plain = true;
+    int32_t exps = kMixed;
+    if (STAGED && n > 0) {
+        exps = __builtin_amdgcn_readfirstlane(unit_meta[0].head.exps);
+        plain = exps != kMixed;
+        for (int i = tid; i < n; i += 256) {
+            const TileHead h = unit_meta[i].head;
+            plain = plain && h.exps == exps && !(h.odd_k | h.odd_v);
+        }
+    }
+    // the keys that some query of the sequence attends; others are zero in the images
+    const int ulo = window_lo(pos0, p.sliding_window);
+    const int uhi = min(pos0 + q_len - 1, p.pm.pos_limit - 1);
 
     // Q^T operand: pieces of Q[query nt*16 + lrow][d = ks*32 + lgrp*8 + 0..7]
     // times the query's own power of two
     half8p qh[NT][KS], ql[NT][KS];
     float qinv[NT];
+    bool qodd[NT];  // the lane's query row holds what the pieces cannot
+    bool any_odd = false;  // some row of the wave does
 #pragma unroll
     for (int nt = 0; nt < NT; nt++) {
         const int lq = wq0 + nt * 16 + lrow;
         const bool ok = lq < q_len;
         const float *qp = p.q + ((int64_t)(row0 + (ok ? lq : 0)) * p.n_heads + head) * D;
         float x[KS][8];
-        uint32_t mx = 0;
+        uint32_t run[KS], top = 0;
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
             const floatx4 a = __builtin_nontemporal_load(reinterpret_cast<const floatx4 *>(qp + ks * 32 + lgrp * 8));
@@ -1641,41 +1525,32 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED>)) void prefill_spl
             for (int j = 0; j < 8; j++) x[ks][j] = ok ? (j < 4 ? a[j & 3] : c[j & 3]) * p.q_mul : 0.0f;
         }
 #pragma unroll
-        for (int ks = 0; ks < KS; ks++)
+        for (int ks = 0; ks < KS; ks++) top = max(top, run[ks] = top_bits(x[ks]));
+        top = umax_rows4(top);
+        const int e = top && top < kInfBits ? exponent_of(top) : kTop;
+        uint32_t bad = top >= kInfBits;
+        qinv[nt] = pow2f(e - kTop);
 #pragma unroll
-            for (int j = 0; j < 8; j++) mx = max(mx, __float_as_uint(x[ks][j]) & 0x7fffffffu);
-        mx = umax_rows4(mx);
-        const float top = __uint_as_float(mx);
-        const bool fits = mx == 0 || (top >= 0x1p-45f && top <= 0x1p45f);  // false for an infinity or a NaN
-        odd = odd || !fits;
-        const int e = mx && fits ? split_exponent<1>(top) : 0;
-        qinv[nt] = pow2f(-e);
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) split8(x[ks], pow2f(e), qh[nt][ks], ql[nt][ks]);
-    }
-    if (STAGED) wait_vm<0>();  // the first tile has landed, so the f32 body may use its place
-    const auto in_f32 = [&]() {
-        constexpr int FT = D == 256 ? 1 : NT;  // d = 256: half a wave's queries at a time, more would spill
-        for (int q = qb0; q < qb0 + qwg; q += 16 * FT * waves_per_head) {
-            __syncthreads();  // the LDS is free
-            prefill_f32_body<D, FT, NW, Q8, CAP>(p, lds, unit, q);
+        for (int ks = 0; ks < KS; ks++) {
+            bad |= run_is_odd(run[ks], top);
+            split8(x[ks], pow2f(kTop - e), qh[nt][ks], ql[nt][ks]);
         }
-    };
-    bool f32 = __syncthreads_or(odd);
-    if (STAGED && f32) {
-        in_f32();
-        return;
+        qodd[nt] = umax_rows4(bad);
+        any_odd = any_odd || __ballot(qodd[nt]);
     }
+    plain = !__syncthreads_or(any_odd || !plain);
 
     floatx4 o[DT][NT];
     float m[NT], lpart[NT];
+    int rexp[NT];  // R: O is in units of 2^(rexp - kTop - kScaleP)
     int qpos[NT], qlo[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; nt++) {
 #pragma unroll
         for (int t = 0; t < DT; t++) o[t][nt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
         lpart[nt] = 0.0f;
-        m[nt] = kMInit;
+        rexp[nt] = kNoExp;
+        m[nt] = kMLowest;  // finite: the first attended key is an ordinary move of the reference
         const int lq = wq0 + nt * 16 + lrow;
         qpos[nt] = lq < q_len ? pos0 + lq : -1;
         qlo[nt] = window_lo(pos0 + lq, p.sliding_window);
@@ -1683,9 +1558,80 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED>)) void prefill_spl
     // keys this wave's queries attend: [wlo, whi]
     const int whi = min(khi, pos0 + wq0 + QW - 1);
     const int wlo = max(klo, window_lo(pos0 + wq0, p.sliding_window));
-    float unit_v = 0.0f;  // O's unit: the scale of the last tile's V (0: none yet)
 
-    auto attend = [&](int i, const uint8_t *kimg, const TileMeta &cur) {
+    // The rare path reads the arguments again: held for it over the tiles that
+    // need none, they and what follows from them crowd the other registers.
+    const auto arguments = [&]() __attribute__((always_inline)) {
+        const PrefillParams *a = (const PrefillParams *)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(a));
+        return a;
+    };
+    const auto head_page = [&](const PrefillParams *a, int k) __attribute__((always_inline)) {
+        return map_page(a->pm, b, min(k, uhi) >> 4) * a->kv.page_stride + (int64_t)kvh * a->kv.head_stride;
+    };
+    // The f32 scores of a tile in place of the pieces' for odd keys and rows.
+    const auto odd_scores = [&](floatx4 (&s)[2][NT], int k0, uint32_t keys) __attribute__((always_inline)) {
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++) {
+            floatx4 e[NT];
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) e[nt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            const int kp = k0 + 16 * mt + lrow;
+            const bool have = kp >= ulo && kp <= uhi;
+            const PrefillParams *a = arguments();
+            const int64_t hb = head_page(a, k0 + 16 * mt);
+#pragma unroll 1
+            for (int step = 0; step < D / 4; step++) {
+                const int d = lgrp * (D / 4) + step;
+                const float kd = have ? k_element<D, Q8>(*a, hb, lrow, d) : 0.0f;
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++) {
+                    const int lq = wq0 + nt * 16 + lrow;
+                    const bool ok = lq < q_len;
+                    const float x = a->q[((int64_t)(row0 + (ok ? lq : 0)) * a->n_heads + head) * D + d] * a->q_mul;
+                    e[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kd, ok ? x : 0.0f, e[nt], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (qodd[nt] || (keys >> (16 * mt + 4 * lgrp + r) & 1)) s[mt][nt][r] = e[nt][r];
+        }
+    };
+    // The products of V's odd values with the probabilities pv (element 4*mt + r
+    // of a lane: key 16*mt + 4*lgrp + r), for the queries that attend them.
+    const auto odd_values = [&](const float (&pv)[NT][8], int k0, uint32_t keys, const TileMeta *meta) __attribute__((always_inline)) {
+        for (; keys; keys &= keys - 1) {
+            const int key = __builtin_ctz(keys), reg = 4 * (key >> 4) + (key & 3);
+            const int kp = k0 + key;
+            const PrefillParams *a = arguments();
+            const int64_t hb = head_page(a, k0 + (key & 16));
+            
+            const float scale = pow2f(kTop - v_exp_of(meta->exps[key]));
+            const LaneV<D, Q8> v(*a, hb, key & 15, lgrp);
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                float mine = pv[nt][0];
+#pragma unroll
+                for (int j = 1; j < 8; j++) mine = reg == j ? pv[nt][j] : mine;
+                const float pk = __shfl(mine, ((key >> 2) & 3) * 16 + lrow);
+                const bool attends = kp >= qlo[nt] && kp <= qpos[nt];
+#pragma unroll
+                for (int t = 0; t < DT; t++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const float x = v(t, r);
+                        const float sum = fmaf(pk, ldexpf(x, kTop + kScaleP - rexp[nt]), o[t][nt][r]);
+                        o[t][nt][r] = attends && v_is_odd(x, scale) ? sum : o[t][nt][r];
+                    }
+            }
+        }
+    };
+
+    // Tile i. `same`: its keys' exponents are those of `exps`, and nothing is odd;
+    // otherwise they are in `meta`.
+    const auto attend = [&](auto same, int i, const uint8_t *kimg, const TileMeta *meta) __attribute__((always_inline)) {
         const int k0 = (tfirst + i) * KT;
         if (k0 > whi || k0 + KT - 1 < wlo) return;  // no query of this wave attends it
 
@@ -1728,132 +1674,208 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED>)) void prefill_spl
         // softmax: as the bf16 kernels' (a lazy maximum), in f32; c undoes the scales
         const bool interior = k0 >= klo && k0 + KT - 1 <= min(khi, pos0 + wq0) &&
                               (p.sliding_window <= 0 || k0 >= window_lo(pos0 + wq0 + QW - 1, p.sliding_window));
-        half8p ph[NT], pl[NT];
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) s[mt][nt][r] = fmaf(x[mt][nt][r], 0x1p-11f, s[mt][nt][r]);
+        float c[NT];  // undoes the scales (powers of two, so where it is done changes no bit)
+        int32_t key[8];
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) c[nt] = same ? pow2f(k_exp_of(exps) - kTop) * qinv[nt] : 1.0f;
+        if constexpr (!same) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) key[j] = meta->exps[(j >> 2) * 16 + 4 * lgrp + (j & 3)];
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) s[mt][nt][r] *= pow2f(k_exp_of(key[4 * mt + r]) - kTop) * qinv[nt];
+            const uint32_t odd_k = __builtin_amdgcn_readfirstlane(meta->head.odd_k);
+            if (odd_k || any_odd) odd_scores(s, k0, odd_k);
+        }
+        float pv[NT][8];
 #pragma unroll
         for (int nt = 0; nt < NT; nt++) {
-            float c = cur.k_inv * qinv[nt];
-            floatx4 col[2] = {s[0][nt] + x[0][nt], s[1][nt] + x[1][nt]};
+            floatx4 col[2] = {s[0][nt], s[1][nt]};
             if constexpr (CAP) {
-                col[0] *= c;
-                col[1] *= c;
-                c = 1.0f;
+                col[0] *= c[nt];
+                col[1] *= c[nt];
+                c[nt] = 1.0f;
             }
             cap_and_mask<CAP>(col, p.softcap, interior, k0 + 4 * lgrp, qpos[nt], qlo[nt], klo, khi);
             float mx = max3f(max3f(col[0][0], col[0][1], col[0][2]), max3f(col[0][3], col[1][0], col[1][1]),
-                             max2f(col[1][2], col[1][3])) * c;
-            if (__ballot(mx - m[nt] > kLazyMax)) {
+                             max2f(col[1][2], col[1][3])) * c[nt];
+            if (__ballot(mx - m[nt] > kLazyF32)) {
                 mx = max_rows4(mx);
-                const bool up = mx - m[nt] > kLazyMax;
+                const bool up = mx - m[nt] > kLazyF32;
                 const float rs = up ? fast_exp2(m[nt] - mx) : 1.0f;
                 m[nt] = up ? mx : m[nt];
 #pragma unroll
                 for (int t = 0; t < DT; t++) o[t][nt] *= rs;
                 lpart[nt] *= rs;
             }
-            const float sub = (float)kSplitP - m[nt];
             float ls = 0.0f;
 #pragma unroll
-            for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const float pv = fast_exp2(fmaf(col[mt][r], c, sub));
-                    ls += pv;
-                    const _Float16 h = (_Float16)pv;
-                    ph[nt][4 * mt + r] = h;
-                    pl[nt][4 * mt + r] = (_Float16)(pv - (float)h);
-                }
+            for (int j = 0; j < 8; j++) {
+                pv[nt][j] = fast_exp2(fmaf(col[j >> 2][j & 3], c[nt], -m[nt]));
+                ls += pv[nt][j];
+            }
             lpart[nt] += ls;
         }
 
-        // O^T += V^T . P^T in V's unit
-        if (cur.v_scale == 0.0f) return;
-        if (cur.v_scale != unit_v) {
-            const float f = unit_v == 0.0f ? 1.0f : cur.v_scale / unit_v;
+        // O^T += V^T . P^T, the probabilities times 2^(E - R)
+        half8p ph[NT], pl[NT];
 #pragma unroll
-            for (int t = 0; t < DT; t++)
+        for (int nt = 0; nt < NT; nt++) {
+            float x[8];
+            if constexpr (same) {
 #pragma unroll
-                for (int nt = 0; nt < NT; nt++) o[t][nt] *= f;
-            unit_v = cur.v_scale;
+                for (int j = 0; j < 8; j++) x[j] = pv[nt][j] * (float)(1 << kScaleP);
+            } else {
+                const int lo = max(qlo[nt], klo), hi = min(qpos[nt], khi);
+                int top = kNoExp;  // of the keys that the row attends
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const int kp = k0 + (j >> 2) * 16 + 4 * lgrp + (j & 3);
+                    top = kp >= lo && kp <= hi ? max(top, v_exp_of(key[j])) : top;
+                }
+                top = (int)umax_rows4((uint32_t)(top - kNoExp)) + kNoExp;
+                if (__ballot(top > rexp[nt] + kLazyExp)) {
+                    const bool up = top > rexp[nt] + kLazyExp;
+                    // (before its first key a row's O is zero)
+                    const float f = up && rexp[nt] != kNoExp ? ldexpf(1.0f, rexp[nt] - top) : 1.0f;
+                    rexp[nt] = up ? top : rexp[nt];
+#pragma unroll
+                    for (int t = 0; t < DT; t++) o[t][nt] *= f;
+                }
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+                    x[j] = pv[nt][j] * ldexpf(1.0f, min(v_exp_of(key[j]) - rexp[nt], kLazyExp) + kScaleP);
+            }
+            split8(x, 1.0f, ph[nt], pl[nt]);
         }
         const uint8_t *vimg = kimg + 128 * D;
+        const auto add_cross = [](floatx4 &to, const floatx4 &x) __attribute__((always_inline)) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) to[r] = fmaf(x[r], 0x1p-11f, to[r]);
+        };
+        floatx4 cross[NT];
 #pragma unroll
         for (int t = 0; t < DT; t++) {
             const uint8_t *src = vimg + ((t * 4 + lgrp) * 16 + lrow) * 16;
             const half8p ah = *reinterpret_cast<const half8p *>(src);
             const half8p al = *reinterpret_cast<const half8p *>(src + 64 * D);
+            floatx4 now[NT];
 #pragma unroll
             for (int nt = 0; nt < NT; nt++)
-                o[t][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, ph[nt], o[t][nt], 0, 0, 0);
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++)
-                o[t][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, pl[nt], o[t][nt], 0, 0, 0);
+                now[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, ph[nt], floatx4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
 #pragma unroll
             for (int nt = 0; nt < NT; nt++)
                 o[t][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, ph[nt], o[t][nt], 0, 0, 0);
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) now[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, pl[nt], now[nt], 0, 0, 0);
+            // the cross terms of the d tile before, whose products are done by now
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                if (t > 0) add_cross(o[t - 1][nt], cross[nt]);
+                cross[nt] = now[nt];
+            }
+        }
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) add_cross(o[DT - 1][nt], cross[nt]);
+        if constexpr (!same) {
+            const uint32_t odd_v = __builtin_amdgcn_readfirstlane(meta->head.odd_v);
+            if (odd_v) odd_values(pv, k0, odd_v, meta);
         }
     };
 
     if constexpr (STAGED) {
-        TileMeta tm = n > 0 ? unit_meta[0] : TileMeta{1.0f, 0.0f};
-        for (int i = 0; i < n; i++) {
-            // this wave's copies of tile i have landed, then every wave's; every
-            // wave is also done with tile i - 1, whose buffer the next copy takes
+        // this wave's copies of tile i have landed, then every wave's; every wave
+        // is also done with tile i - 1, whose buffer the next copy takes
+        const auto arrive = [&](int i) __attribute__((always_inline)) {
             wait_vm<0>();
             __syncthreads();
             if (i + 1 < n) issue(i + 1);
-            const TileMeta cur = tm;
-            tm = unit_meta[min(i + 1, n - 1)];
-            attend(i, lds + (i & 1) * IMG, cur);
+        };
+        if (plain) {
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) rexp[nt] = v_exp_of(exps);
+            for (int i = 0; i < n; i++) {
+                arrive(i);
+                attend(std::true_type{}, i, lds + (i & 1) * IMG, nullptr);
+            }
+        } else {
+            const TileMeta *metas = reinterpret_cast<const TileMeta *>(lds + METAS);
+            if (n > 0) issue_meta(0);
+            for (int i = 0; i < n; i++) {
+                arrive(i);
+                if (i + 1 < n) issue_meta(i + 1);
+                attend(std::false_type{}, i, lds + (i & 1) * IMG, metas + (i & 1));
+            }
         }
-    } else if (n > 0 && !f32) {
+    } else if (n > 0) {
         SplitAux<D, Q8> &aux = *reinterpret_cast<SplitAux<D, Q8> *>(lds + IMG);
-        // the keys that a staged tile would hold: what any query of the sequence attends
-        const int ulo = window_lo(pos0, p.sliding_window);
-        const int uhi = min(pos0 + q_len - 1, p.pm.pos_limit - 1);
         constexpr bool AHEAD = D < 256;
         SplitTile<D, Q8> tile;
         tile.fetch(p, b, kvh, tfirst * KT, ulo, uhi);
-        for (int i = 0; i < n; i++) {
+        if (tid < 2) aux.odd[tid] = 0;
+        __syncthreads();
+        const auto put = [&](int base) {
+            uint8_t *to = lds + base;
+            return [to](int j, const half8p &hi, const half8p &lo) {
+                *reinterpret_cast<half8p *>(to + j * 16) = hi;
+                *reinterpret_cast<half8p *>(to + 64 * D + j * 16) = lo;
+            };
+        };
+        // tile i, ready for every wave
+        const auto arrive = [&](int i) __attribute__((always_inline)) {
             const int k0 = (tfirst + i) * KT;
+            if (i > 0) __syncthreads();  // its place is free
             if (!AHEAD && i > 0) tile.fetch(p, b, kvh, k0, ulo, uhi);
-            tile.convert(aux, k0, ulo, uhi, [&](int j, const half8p &kh, const half8p &kl, const half8p &vh, const half8p &vl) {
-                *reinterpret_cast<half8p *>(lds + j * 16) = kh;
-                *reinterpret_cast<half8p *>(lds + 64 * D + j * 16) = kl;
-                *reinterpret_cast<half8p *>(lds + 128 * D + j * 16) = vh;
-                *reinterpret_cast<half8p *>(lds + 192 * D + j * 16) = vl;
-            });
+            tile.convert(aux, k0, ulo, uhi, put(0), put(128 * D));
             __syncthreads();
-            const TileMeta cur = aux.meta;
-            if (cur.k_inv != cur.k_inv) {
-                f32 = true;
-                break;
-            }
             if (AHEAD && i + 1 < n) tile.fetch(p, b, kvh, k0 + KT, ulo, uhi);
-            attend(i, lds, cur);
-            __syncthreads();  // before the next tile takes its place
+        };
+        int i = 0;
+        bool here = false;  // tile i is ready
+        for (; i < n && plain; i++) {
+            arrive(i);
+            if (i == 0) exps = __builtin_amdgcn_readfirstlane(aux.meta.head.exps);
+            here = exps == kMixed || __builtin_amdgcn_readfirstlane(aux.meta.head.exps) != exps ||
+                   __builtin_amdgcn_readfirstlane(aux.meta.head.odd_k | aux.meta.head.odd_v);
+            if (here) break;
+            attend(std::true_type{}, i, lds, nullptr);
+        }
+        // (a row that has attended a key has moved its maximum)
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++)
+            if (i > 0 && m[nt] != kMLowest) rexp[nt] = v_exp_of(exps);
+        for (; i < n; i++, here = false) {
+            if (!here) arrive(i);
+            attend(std::false_type{}, i, lds, &aux.meta);
         }
     }
 
-    if (!STAGED && f32) {
-        in_f32();
-        return;
-    }
-
     // Output rows through LDS, as the staged bf16 kernel writes them
-    constexpr int SROW = D + 4;
-    static_assert(NW * 16 * SROW * 4 <= LDS, "output staging fits");
     __syncthreads();
     float *stage = reinterpret_cast<float *>(lds) + wave * 16 * SROW;
     constexpr int LPR = D / 4;    // lanes per row (16 bytes each)
     constexpr int RPI = 64 / LPR;  // rows per store instruction
-    const float unscale = unit_v == 0.0f ? 1.0f : 1.0f / unit_v;
 #pragma unroll
     for (int nt = 0; nt < NT; nt++) {
         const float lt = sum_rows4(lpart[nt]);
-        const float inv = lt > 0.0f ? 1.0f / lt * unscale : 0.0f;
+        const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
+        const int unit_exp = rexp[nt] == kNoExp ? 0 : rexp[nt] - kTop - kScaleP;
 #pragma unroll
-        for (int t = 0; t < DT; t++)
-            *reinterpret_cast<floatx4 *>(stage + lrow * SROW + 16 * t + 4 * lgrp) = o[t][nt] * inv;
+        for (int t = 0; t < DT; t++) {
+            floatx4 x;
+#pragma unroll
+            for (int r = 0; r < 4; r++) x[r] = ldexpf(o[t][nt][r] * inv, unit_exp);
+            *reinterpret_cast<floatx4 *>(stage + lrow * SROW + 16 * t + 4 * lgrp) = x;
+        }
 #pragma unroll
         for (int k = 0; k < 16 / RPI; k++) {
             const int r = k * RPI + lane / LPR;
