@@ -1269,41 +1269,97 @@ struct SplitTile {
     }
 };
 
-// Grid (tile, (sequence, KV head) pair), 256 threads.
-template <int D, bool Q8>
-__global__ __launch_bounds__(256) void stage_split_kernel(const PrefillParams p, uint8_t *img, TileMeta *meta,
-                                                          int n_tiles, int pair0) {
-    const int t = blockIdx.x;
-    const int pair = pair0 + blockIdx.y;
-    const int b = pair / p.n_kv_heads;
-    const int kvh = pair - b * p.n_kv_heads;
-    const int row0 = p.q_start[b];
-    const int q_len = min(max(p.q_start[b + 1] - row0, 0), p.max_q_len);
-    if (q_len == 0) return;
-    const int pos0 = p.pos_offset[b];
-    const int khi = min(pos0 + q_len - 1, p.pm.pos_limit - 1);
-    const int klo = window_lo(pos0, p.sliding_window);
-    const int k0 = t * KT;
-    if (khi < klo || k0 > khi || k0 + KT - 1 < klo) return;  // a tile no query of the sequence reads
+// The tiles that some query of sequence b attends.
+struct SeqTiles {
+    int lo, hi;        // the keys: [lo, hi], hi < 0 if there are none
+    int first, count;  // their tiles
+    __device__ __forceinline__ SeqTiles(const PrefillParams &p, int b) {
+        const int q_len = min(max(p.q_start[b + 1] - p.q_start[b], 0), p.max_q_len);
+        const int pos0 = p.pos_offset[b];
+        lo = window_lo(pos0, p.sliding_window);
+        hi = q_len > 0 ? min(pos0 + q_len - 1, p.pm.pos_limit - 1) : -1;
+        first = lo / KT;
+        count = hi >= lo ? hi / KT - first + 1 : 0;
+    }
+};
 
+// Where the tile images of a (sequence, KV head) pair are. `start` null: every
+// pair has `stride` places. Else the attended tiles of all pairs are numbered one
+// after the other, start[b] being the first of sequence b's, and taken in rounds:
+// a pair belongs to the round in whose `span` numbers its first tile falls, and
+// may run past them by up to `over`. A longer pair, or one past the last round,
+// has none.
+struct Images {
+    uint8_t *img;
+    TileMeta *meta;
+    const int64_t *start;
+    int stride, span, over, round, rounds;
+    __device__ __forceinline__ bool here(int b, int kvh, int count) const {
+        if (!start) return true;
+        const int64_t at = start[b] + (int64_t)kvh * count - (int64_t)round * span;
+        return at >= 0 && at < span && count <= over;
+    }
+    __device__ __forceinline__ bool nowhere(int b, int kvh, int count) const {
+        return !start || start[b] + (int64_t)kvh * count >= (int64_t)rounds * span || count > over;
+    }
+    __device__ __forceinline__ int64_t first(int b, int kvh, int n_kv_heads, int count) const {
+        return start ? start[b] + (int64_t)kvh * count - (int64_t)round * span
+                     : ((int64_t)b * n_kv_heads + kvh) * stride;
+    }
+};
+
+// start[b] of every sequence. One workgroup; a call that has a place for every
+// tile its storage could have it attend does without.
+__global__ __launch_bounds__(1024) void image_start_kernel(const PrefillParams p, int n_seqs, int64_t *start) {
+    __shared__ int64_t sum[1024];
+    int64_t before = 0;
+    for (int b0 = 0; b0 < n_seqs; b0 += 1024) {
+        const int b = b0 + threadIdx.x;
+        const int64_t mine = b < n_seqs ? (int64_t)SeqTiles(p, b).count * p.n_kv_heads : 0;
+        sum[threadIdx.x] = mine;
+        for (int d = 1; d < 1024; d *= 2) {
+            __syncthreads();
+            const int64_t x = (int)threadIdx.x >= d ? sum[threadIdx.x - d] : 0;
+            __syncthreads();
+            sum[threadIdx.x] += x;
+        }
+        __syncthreads();
+        if (b < n_seqs) start[b] = before + sum[threadIdx.x] - mine;
+        before += sum[1023];
+        __syncthreads();
+    }
+}
+
+// Grid (sequence, slice): the workgroups of a sequence take its (KV head, tile)
+// pairs in turn, as many as it has. 256 threads.
+template <int D, bool Q8>
+__global__ __launch_bounds__(256) void stage_split_kernel(const PrefillParams p, const Images im) {
+    const int b = blockIdx.x;
+    const SeqTiles seq(p, b);
     __shared__ __attribute__((aligned(16))) SplitAux<D, Q8> aux;
-    SplitTile<D, Q8> tile;
-    tile.fetch(p, b, kvh, k0, klo, khi);
     if (threadIdx.x < 2) aux.odd[threadIdx.x] = 0;
-    __syncthreads();
-    const int64_t at = (int64_t)blockIdx.y * n_tiles + t;
-    uint8_t *dst = img + at * kSplitImage<D>;
-    const auto put = [&](uint8_t *to) {
-        return [to](int i, const half8p &hi, const half8p &lo) {
-            *reinterpret_cast<half8p *>(to + i * 16) = hi;
-            *reinterpret_cast<half8p *>(to + 64 * D + i * 16) = lo;
+    for (int item = blockIdx.y; item < seq.count * p.n_kv_heads; item += gridDim.y) {
+        const int kvh = item / seq.count;
+        const int t = item - kvh * seq.count;
+        if (!im.here(b, kvh, seq.count)) continue;
+        const int k0 = (seq.first + t) * KT;
+        SplitTile<D, Q8> tile;
+        tile.fetch(p, b, kvh, k0, seq.lo, seq.hi);
+        __syncthreads();  // aux is free
+        const int64_t at = im.first(b, kvh, p.n_kv_heads, seq.count) + t;
+        uint8_t *dst = im.img + at * kSplitImage<D>;
+        const auto put = [](uint8_t *to) {
+            return [to](int i, const half8p &hi, const half8p &lo) {
+                *reinterpret_cast<half8p *>(to + i * 16) = hi;
+                *reinterpret_cast<half8p *>(to + 64 * D + i * 16) = lo;
+            };
         };
-    };
-    tile.convert(aux, k0, klo, khi, put(dst), put(dst + 128 * D));
-    __syncthreads();
-    constexpr int WORDS = sizeof(TileMeta) / 4;
-    if (threadIdx.x < WORDS)
-        reinterpret_cast<uint32_t *>(meta + at)[threadIdx.x] = reinterpret_cast<const uint32_t *>(&aux.meta)[threadIdx.x];
+        tile.convert(aux, k0, seq.lo, seq.hi, put(dst), put(dst + 128 * D));
+        __syncthreads();
+        constexpr int WORDS = sizeof(TileMeta) / 4;
+        if (threadIdx.x < WORDS)
+            reinterpret_cast<uint32_t *>(im.meta + at)[threadIdx.x] = reinterpret_cast<const uint32_t *>(&aux.meta)[threadIdx.x];
+    }
 }
 
 // The staging launch of the bf16 path.
@@ -1424,9 +1480,7 @@ constexpr int kSplitOccupancy = !STAGED ? (D == 64 ? 2 : 1) : (D == 64 ? 4 - NT 
 
 template <int D, bool Q8, bool CAP, bool STAGED, int NT>
 __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill_split_kernel(const PrefillParams p,
-                                                                                const uint8_t *img,
-                                                                                const TileMeta *meta, int n_tiles,
-                                                                                int pair0) {
+                                                                                                const Images im) {
     constexpr int NW = 4;
     constexpr int QW = 16 * NT;
     constexpr int KS = D / 32;
@@ -1440,12 +1494,11 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill
     __shared__ __attribute__((aligned(16))) uint8_t lds[LDS];
 
     const int n_hgrp = p.group / p.hpw;
-    const int unit = pair0 * n_hgrp + (int)blockIdx.x;
-    const int pair = unit / n_hgrp;
+    const int pair = (int)blockIdx.x / n_hgrp;
     const int b = pair / p.n_kv_heads;
     const int kvh = pair - b * p.n_kv_heads;
-    const int hgrp = unit - pair * n_hgrp;
-    const int qblk = p.n_qblocks - 1 - (int)blockIdx.y;
+    const int hgrp = (int)blockIdx.x - pair * n_hgrp;
+    const int qblk = p.n_qblocks - 1 - (int)(blockIdx.z * gridDim.y + blockIdx.y);
     const int waves_per_head = NW / p.hpw;
     const int qwg = QW * waves_per_head;
 
@@ -1453,7 +1506,9 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill
     const int q_len = min(max(p.q_start[b + 1] - row0, 0), p.max_q_len);
     const int pos0 = p.pos_offset[b];
     const int qb0 = qblk * qwg;
-    if (qb0 >= q_len) return;
+    if (qblk < 0 || qb0 >= q_len) return;
+    const SeqTiles seq(p, b);
+    if (STAGED ? !im.here(b, kvh, seq.count) : !im.nowhere(b, kvh, seq.count)) return;  // another launch's
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -1468,8 +1523,11 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill
     const int klo = window_lo(pos0 + qb0, p.sliding_window);
     const int tfirst = klo / KT;
     const int n = khi >= klo ? khi / KT - tfirst + 1 : 0;
-    const TileMeta *unit_meta = meta + (int64_t)(pair - pair0) * n_tiles + tfirst;
-    const uint8_t *unit_img = img + ((int64_t)(pair - pair0) * n_tiles + tfirst) * IMG;
+    // the keys that some query of the sequence attends; others are zero in the images
+    const int ulo = seq.lo, uhi = seq.hi;
+    const int64_t first = STAGED ? im.first(b, kvh, p.n_kv_heads, seq.count) + tfirst - seq.first : 0;
+    const TileMeta *unit_meta = im.meta + first;
+    const uint8_t *unit_img = im.img + first * IMG;
     const uint32_t ring = __builtin_amdgcn_readfirstlane(
         (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)&lds[0]);
     auto issue = [&](int i) {
@@ -1500,9 +1558,6 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill
             plain = plain && h.exps == exps && !(h.odd_k | h.odd_v);
         }
     }
-    // the keys that some query of the sequence attends; others are zero in the images
-    const int ulo = window_lo(pos0, p.sliding_window);
-    const int uhi = min(pos0 + q_len - 1, p.pm.pos_limit - 1);
 
     // Q^T operand: pieces of Q[query nt*16 + lrow][d = ks*32 + lgrp*8 + 0..7]
     // times the query's own power of two
@@ -1942,78 +1997,101 @@ int launch_bf16(gla_ctx *ctx, const PrefillParams &prm, dim3 grid) {
     return GLA_OK;
 }
 
-// Tile images an fp32 prefill may hold in scratch; a call with more (sequence,
-// KV head) pairs runs in several rounds over them.
-constexpr size_t kSplitScratch = (size_t)1 << 30;
-// Query rows of a call's longest sequence up to which workgroups convert their
-// own tiles: the second launch costs a short prompt more than the repeated
-// conversion, but each row block converts the whole past again. One sequence,
-// us per call, unstaged / staged: from position 0, d = 128 20 rows 7.7 / 12.0,
-// 90 rows 12.6 / 16.1, 150 rows 17.8 / 19.7; d = 64 20 rows 5.6 / 9.2, 100 rows
-// 11.0 / 13.5; d = 256 with the soft-cap 20 rows 11.4 / 17.3, 100 rows 27.9 /
-// 30.6. After 1,000 cached positions, d = 128: 100 rows 93 / 71.
-constexpr int kUnstagedRows = 96;
+// Bytes of tile images that an fp32 prefill may hold in scratch, and up to which
+// it keeps a place for every tile that the storage could have it attend. Above
+// that the device numbers the tiles that it does attend, and the host, which
+// knows the storage's length but not the contexts, launches the rounds that the
+// longest ones would need, up to kRounds; an empty one costs some 5 us. 64 prompts of 200
+// rows in a storage of 32,768 positions 234 us, of 200 positions 194.
+constexpr size_t kSplitScratch = (size_t)1 << 30, kSplitDirect = (size_t)256 << 20;
+constexpr int kRounds = 4;
+// Query rows of a call's longest sequence, and tiles of its storage, up to which
+// workgroups convert their own tiles: the second launch costs such a call more than
+// the repeated conversion. One sequence, us per call, unstaged / staged: from
+// position 0, d = 128 20 rows 9.2 / 11.5, 90 rows 15.5 / 14.5; d = 64 20 rows 7.1 /
+// 9.4; d = 256 20 rows 13.4 / 15.2; after 300 cached positions 20 rows 36 / 22,
+// after 4,000 387 / 151.
+constexpr int kUnstagedRows = 32;
+constexpr int kUnstagedTiles = 4;
 
-// fp32 prefill: the tile images of as many (sequence, KV head) pairs as the
-// scratch takes, then their attention. A call of few query blocks has each
-// workgroup convert its own tiles instead (the same bits), and so has one whose
-// scratch cannot be had: it would have to grow during a capture, the device is
-// full, or one pair's images alone pass the bound.
-template <int D, bool Q8, bool CAP>
-int launch_split(gla_ctx *ctx, PrefillParams prm, int n_pairs, int n_hgrp, int n_tiles) {
-    const size_t per = (size_t)n_tiles * (kSplitImage<D> + sizeof(TileMeta));
-    uint8_t *img = nullptr;
-    int round = n_pairs;
-    if (prm.max_q_len > kUnstagedRows && n_tiles > 0 && per <= kSplitScratch) {
-        round = (int)std::min<size_t>({(size_t)n_pairs, kSplitScratch / per, (size_t)65535});
-        void *scr = nullptr;
-        if (ensure_scratch(ctx, round * per, &scr) == GLA_OK) {
-            img = (uint8_t *)scr;
-        } else {
-            clear_error();
-            (void)hipGetLastError();
-            round = n_pairs;
-        }
-    }
-    // (the few rows of an unstaged call are spread over the most waves)
-    const int nt = img ? wave_tiles(ctx, prm, std::min(round, n_pairs) * n_hgrp) : 1;
-    prm.n_qblocks = wg_blocks(prm, nt);
-    if (prm.n_qblocks > 65535) return set_error(GLA_ERR_INVALID, "prefill: %d query blocks > 65535", prm.n_qblocks);
-    if (!img) {
-        hipLaunchKernelGGL((prefill_split_kernel<D, Q8, CAP, false, 1>), dim3(n_pairs * n_hgrp, prm.n_qblocks), dim3(256),
-                           0, ctx->stream, prm, (const uint8_t *)nullptr, (const TileMeta *)nullptr, n_tiles, 0);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "prefill_split_kernel launch: %s", hipGetErrorString(e));
-        return GLA_OK;
-    }
-    TileMeta *meta = reinterpret_cast<TileMeta *>(img + (size_t)round * n_tiles * kSplitImage<D>);
-    for (int p0 = 0; p0 < n_pairs; p0 += round) {
-        const int np = std::min(round, n_pairs - p0);
-        hipLaunchKernelGGL((stage_split_kernel<D, Q8>), dim3(n_tiles, np), dim3(256), 0, ctx->stream, prm, img, meta,
-                           n_tiles, p0);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "stage_split_kernel launch: %s", hipGetErrorString(e));
-        const dim3 grid(np * n_hgrp, prm.n_qblocks);
-        if (nt == 1)
-            hipLaunchKernelGGL((prefill_split_kernel<D, Q8, CAP, true, 1>), grid, dim3(256), 0, ctx->stream, prm,
-                               (const uint8_t *)img, (const TileMeta *)meta, n_tiles, p0);
-        else
-            hipLaunchKernelGGL((prefill_split_kernel<D, Q8, CAP, true, 2>), grid, dim3(256), 0, ctx->stream, prm,
-                               (const uint8_t *)img, (const TileMeta *)meta, n_tiles, p0);
-        e = hipGetLastError();
-        if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "prefill_split_kernel launch: %s", hipGetErrorString(e));
-    }
+template <int D, bool Q8, bool CAP, bool STAGED, int NT>
+int launch_split_as(gla_ctx *ctx, PrefillParams prm, int n_units, const Images &im) {
+    prm.n_qblocks = wg_blocks(prm, NT);
+    const int y = std::min(prm.n_qblocks, 65535);
+    hipLaunchKernelGGL((prefill_split_kernel<D, Q8, CAP, STAGED, NT>), dim3(n_units, y, (prm.n_qblocks - 1) / y + 1),
+                       dim3(256), 0, ctx->stream, prm, im);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "prefill_split_kernel launch: %s", hipGetErrorString(e));
     return GLA_OK;
 }
 
+// fp32 prefill: the images of the tiles that its sequences attend, then the
+// attention. A call of few rows over a small storage has each workgroup convert
+// its own tiles instead (the same bits), and so have the pairs that no round
+// takes and a call whose scratch cannot be had (it would have to grow during a
+// capture, or the device is full): 4 x 2,048 rows 944 us, 997 rows 105 us.
+template <int D, bool Q8, bool CAP>
+int launch_split(gla_ctx *ctx, const PrefillParams &prm, int n_seqs, int n_hgrp, int n_tiles) {
+    const int n_pairs = n_seqs * prm.n_kv_heads, n_units = n_pairs * n_hgrp;
+    // tiles that one sequence can attend
+    if (prm.sliding_window > 0)
+        n_tiles = (int)std::min<int64_t>(n_tiles, ((int64_t)prm.max_q_len + prm.sliding_window - 2) / KT + 2);
+    constexpr size_t per = kSplitImage<D> + sizeof(TileMeta);
+    const bool few = prm.max_q_len <= kUnstagedRows && n_tiles <= kUnstagedTiles;
+    Images im{};
+    im.rounds = 1;
+    bool all_placed = true;
+    if (!few && n_tiles > 0) {
+        const size_t all = (size_t)n_pairs * n_tiles;
+        const bool direct = all * per <= kSplitDirect;
+        const size_t places = std::min(all, kSplitScratch / per);
+        const size_t start_bytes = direct ? 0 : (size_t)n_seqs * sizeof(int64_t);
+        void *scr = nullptr;
+        if (ensure_scratch(ctx, places * per + start_bytes, &scr) == GLA_OK) {
+            im.img = (uint8_t *)scr;
+            im.meta = reinterpret_cast<TileMeta *>(im.img + places * kSplitImage<D>);
+            im.stride = n_tiles;
+            if (!direct) {
+                int64_t *start = reinterpret_cast<int64_t *>(im.meta + places);
+                im.start = start;
+                // (all of them in one round, or a quarter of the places for the last pair's overrun)
+                im.over = (int)(places == all ? (size_t)n_tiles : places / 4);
+                im.span = (int)(places == all ? all : places - im.over);
+                const size_t rounds = (all - 1) / im.span + 1;
+                im.rounds = (int)std::min<size_t>(rounds, kRounds);
+                all_placed = rounds <= kRounds && n_tiles <= im.over;
+                hipLaunchKernelGGL(image_start_kernel, dim3(1), dim3(1024), 0, ctx->stream, prm, n_seqs, start);
+                const hipError_t e = hipGetLastError();
+                if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "image_start_kernel launch: %s", hipGetErrorString(e));
+            }
+        } else {
+            clear_error();
+            (void)hipGetLastError();
+        }
+    }
+    if (!im.img) return launch_split_as<D, Q8, CAP, false, 1>(ctx, prm, n_units, im);
+    // one tile a workgroup, up to some eight workgroups per CU
+    const int64_t items = (int64_t)n_tiles * prm.n_kv_heads;
+    const int slices = (int)std::min<int64_t>({items, std::max(64, 8 * ctx->n_cu / n_seqs), 65535});
+    for (; im.round < im.rounds; im.round++) {
+        hipLaunchKernelGGL((stage_split_kernel<D, Q8>), dim3(n_seqs, slices), dim3(256), 0, ctx->stream, prm, im);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return set_error(GLA_ERR_KERNEL, "stage_split_kernel launch: %s", hipGetErrorString(e));
+        const int rc = wave_tiles(ctx, prm, n_units) == 1 ? launch_split_as<D, Q8, CAP, true, 1>(ctx, prm, n_units, im)
+                                                          : launch_split_as<D, Q8, CAP, true, 2>(ctx, prm, n_units, im);
+        if (rc != GLA_OK) return rc;
+    }
+    return all_placed ? GLA_OK : launch_split_as<D, Q8, CAP, false, 1>(ctx, prm, n_units, im);
+}
+
 template <int D>
-int launch_f32(gla_ctx *ctx, bool q8, const PrefillParams &prm, int n_pairs, int n_hgrp, int n_tiles) {
+int launch_f32(gla_ctx *ctx, bool q8, const PrefillParams &prm, int n_seqs, int n_hgrp, int n_tiles) {
     const bool cap = prm.softcap > 0.0f;
     if (q8)
-        return cap ? launch_split<D, true, true>(ctx, prm, n_pairs, n_hgrp, n_tiles)
-                   : launch_split<D, true, false>(ctx, prm, n_pairs, n_hgrp, n_tiles);
-    return cap ? launch_split<D, false, true>(ctx, prm, n_pairs, n_hgrp, n_tiles)
-               : launch_split<D, false, false>(ctx, prm, n_pairs, n_hgrp, n_tiles);
+        return cap ? launch_split<D, true, true>(ctx, prm, n_seqs, n_hgrp, n_tiles)
+                   : launch_split<D, true, false>(ctx, prm, n_seqs, n_hgrp, n_tiles);
+    return cap ? launch_split<D, false, true>(ctx, prm, n_seqs, n_hgrp, n_tiles)
+               : launch_split<D, false, false>(ctx, prm, n_seqs, n_hgrp, n_tiles);
 }
 
 }  // namespace
@@ -2086,14 +2164,14 @@ int launch_prefill(gla_ctx *ctx, const PrefillLaunch &a) {
             return a.q8 ? launch_bf16<256, true>(ctx, prm, grid) : launch_bf16<256, false>(ctx, prm, grid);
         }
     }
-    const int n_pairs = a.n_seqs * a.n_kv_heads, n_hgrp = group / hpw;
+    const int n_hgrp = group / hpw;
     switch (D) {
     case 64:
-        return launch_f32<64>(ctx, a.q8, prm, n_pairs, n_hgrp, n_tiles);
+        return launch_f32<64>(ctx, a.q8, prm, a.n_seqs, n_hgrp, n_tiles);
     case 128:
-        return launch_f32<128>(ctx, a.q8, prm, n_pairs, n_hgrp, n_tiles);
+        return launch_f32<128>(ctx, a.q8, prm, a.n_seqs, n_hgrp, n_tiles);
     default:
-        return launch_f32<256>(ctx, a.q8, prm, n_pairs, n_hgrp, n_tiles);
+        return launch_f32<256>(ctx, a.q8, prm, a.n_seqs, n_hgrp, n_tiles);
     }
 }
 

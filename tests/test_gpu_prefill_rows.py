@@ -174,3 +174,34 @@ def test_scores_near_the_end_of_f32(backend, d, exponent, tiles_apart):
             w = np.exp2(s[:r + 1] - s[:r + 1].max())
             want = w @ vh[:r + 1] / w.sum()
             assert np.abs(got[r, h] - want).max() <= 1e-5, (h, r)
+
+
+@pytest.mark.parametrize("d,H,Hkv,seqs,cached", [(64, 8, 8, 16, 65000), (128, 8, 8, 5, 70000), (256, 4, 4, 3, 70000)])
+def test_images_in_rounds_and_none(backend, d, H, Hkv, seqs, cached):
+    """Contexts whose tile images pass the scratch bound several times: taken in rounds, and at d = 64 the last
+    sequences past the last round convert their own tiles. Each has the bits of itself alone, and what it attends:
+    every page of the table is one of a few physical pages, so 64 bits need the few."""
+    page, pool_pages, rows = 16, 24, [35, 1, 20, 40]
+    pool = backend.create_page_pool(pool_pages, Hkv, d, "f32")
+    n = pool_pages * page
+    k, v = synth.normal_rows(101, n, Hkv * d), synth.normal_rows(102, n, Hkv * d)
+    pool.write_rows(np.arange(n, dtype=np.int64), k, v)
+    lens = [rows[b % len(rows)] for b in range(seqs)]
+    pages = (cached + max(lens) + page - 1) // page
+    table = np.random.default_rng(103).integers(0, pool_pages, (seqs, pages)).astype(np.int32)
+    q = synth.normal(104, (sum(lens), H, d))
+    start = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    both = run_prefill(backend, pool, q, start, [cached] * seqs, H, 0.1, table=table)
+    for b in range(seqs):
+        part = slice(start[b], start[b + 1])
+        alone = run_prefill(backend, pool, q[part], [0, lens[b]], [cached], H, 0.1, table=table[b:b + 1])
+        assert _same(alone, both[part]), b
+        if b in (0, seqs - 1):  # the last row: each physical slot as often as the table names its page
+            end = cached + lens[b]
+            at = table[b, np.arange(end) // page].astype(np.int64) * page + np.arange(end) % page
+            for h in (0, H - 1):
+                cols = slice(h * Hkv // H * d, (h * Hkv // H + 1) * d)
+                want = attention_f64(q[start[b + 1] - 1, h], k[at][:, cols], v[at][:, cols],
+                                     np.float64(np.float32(0.1)))
+                assert np.abs(both[start[b + 1] - 1, h] - want).max() <= 1e-5, (b, h)
+    pool.destroy()
