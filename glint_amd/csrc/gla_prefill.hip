@@ -887,8 +887,12 @@ __global__ __launch_bounds__(kBf16sWaves<D> * 64, kBf16sOccupancy<D>) void prefi
 // What the pieces cannot hold is named per key ("odd"): infinities and NaN, K
 // with a run of 8 dims below 2^-20 of its largest value, V's values below kSmall
 // (scaled). The scores of an odd key, or of a query row that is odd in the same
-// way, come from the f32 MFMA; odd V values are zero in the image, and their
-// products are added in f32 for the rows that attend them.
+// way, come from the f32 MFMA. Odd V values are zero in the image; the small
+// ones' products are added by the f32 MFMA, the others' for the rows that attend
+// them. us per call of 4 x 2,048 rows, 32/8 heads, d = 128: 394 where nothing
+// differs, 480 where the keys' exponents differ, 510 with a NaN in V, 1,400 with every
+// 16th dim of V at 2^-34 of the others, 2,200 with eight dims of every key at 2^-30
+// (f32 MFMAs for everything: 1,080).
 typedef _Float16 half8p __attribute__((ext_vector_type(8)));
 
 constexpr float kMLowest = -3.402823466e38f;  // a row's maximum before its first key
@@ -906,12 +910,13 @@ constexpr int kSplitImage = 256 * D;
 // What the attention needs to know of a tile.
 struct TileHead {
     int32_t exps;           // the keys' exponents (key_exps); kMixed: they differ
-    uint32_t odd_k, odd_v;  // odd keys, a bit each
+    uint32_t odd_k;         // odd keys, a bit each: of K,
+    uint32_t bad_v, small_v;  // of V by an infinity or a NaN, by a small value
 };
 struct TileMeta {
     TileHead head;
     int32_t exps[KT];  // by key, where it is in range
-    uint32_t pad[29];  // 256 bytes: four for each lane of a wave
+    uint32_t pad[28];  // 256 bytes: four for each lane of a wave
 };
 static_assert(sizeof(TileMeta) == 256, "one 4-byte copy per lane");
 constexpr int32_t kMixed = -1;
@@ -975,31 +980,35 @@ __device__ __forceinline__ uint32_t umax_group(uint32_t x) {
     return x;
 }
 
-// One element of a cached K row (page and head offset in hb).
+// Four values of a cached K row from d on (page and head offset in hb).
 template <int D, bool Q8>
-__device__ __forceinline__ float k_element(const PrefillParams &p, int64_t hb, int slot, int d) {
+__device__ __forceinline__ floatx4 k_values4(const PrefillParams &p, int64_t hb, int slot, int d) {
     if constexpr (Q8) {
         const uint16_t sc = reinterpret_cast<const uint16_t *>(p.kv.ks + hb)[q8ks_off(slot, d >> 5, D)];
-        return (float)((int)p.kv.k[hb + q8k_off(slot, d, D)] - 128) * __half2float(__ushort_as_half(sc));
+        const uint32_t w = *reinterpret_cast<const uint32_t *>(p.kv.k + hb + q8k_off(slot, d, D));
+        floatx4 x;
+#pragma unroll
+        for (int j = 0; j < 4; j++) x[j] = (float)((int)((w >> (8 * j)) & 0xff) - 128) * __half2float(__ushort_as_half(sc));
+        return x;
     } else {
-        return reinterpret_cast<const float *>(p.kv.k + hb + (int64_t)slot * p.kv.row_stride)[d];
+        return *reinterpret_cast<const floatx4 *>(p.kv.k + hb + (int64_t)slot * p.kv.row_stride + 4 * (int64_t)d);
     }
 }
 
-// V of a cached row at the dims 16*t + 4*lgrp + r that a lane's O holds. (The
+// V of a cached row at the dims 16*t + d0 + r, d0 + r < 16. (The
 // addresses are opaque so that nothing of them is kept in registers over the
 // tiles that need none.)
 template <int D, bool Q8>
 struct LaneV {
     const uint8_t *v;
     const uint16_t *scale;
-    __device__ __forceinline__ LaneV(const PrefillParams &p, int64_t hb, int slot, int lgrp) {
+    __device__ __forceinline__ LaneV(const PrefillParams &p, int64_t hb, int slot, int d0) {
         if constexpr (Q8) {
-            v = p.kv.v + hb + q8v_off(slot, 4 * lgrp, D);
+            v = p.kv.v + hb + q8v_off(slot, d0, D);
             scale = reinterpret_cast<const uint16_t *>(p.kv.vs + hb) + slot * (D / 32);
             asm volatile("" : "+v"(scale));
         } else {
-            v = p.kv.v + hb + (int64_t)slot * p.kv.row_stride + 16 * lgrp;
+            v = p.kv.v + hb + (int64_t)slot * p.kv.row_stride + 4 * d0;
             scale = nullptr;
         }
         asm volatile("" : "+v"(v));
@@ -1014,9 +1023,10 @@ struct LaneV {
 };
 
 // Whether the image holds V value v of a key with scale 2^(kTop - e) as zero.
-__device__ __forceinline__ bool v_is_odd(float v, float scale) {
+__device__ __forceinline__ bool v_is_bad(float v) { return !(fabsf(v) < INFINITY); }
+__device__ __forceinline__ bool v_is_small(float v, float scale) {
     const float t = fabsf(v) * scale;
-    return !(t < INFINITY) || (t < kSmall && t > 0.0f);
+    return t < kSmall && t > 0.0f;
 }
 
 // One 32-key tile of a (sequence, KV head) pair on its way from the cache to
@@ -1034,8 +1044,8 @@ __device__ __forceinline__ int v_piece_dim(int i) { return 16 * (i >> 6) + (i & 
 template <int D, bool Q8>
 struct SplitAux {
     int k_exp[KT], v_exp[KT];
-    uint32_t odd[2];
-    uint32_t pad[2];
+    uint32_t odd[3];  // TileHead's masks
+    uint32_t pad[1];
     TileMeta meta;
     float v[Q8 ? 1 : KT][Q8 ? 4 : D + 4];  // scaled rows of V, read back along the keys
 };
@@ -1170,7 +1180,9 @@ struct SplitTile {
                 const bool small = top && (threadIdx.x < 32 ? low + (13u << 23) < top
                                                             : __uint_as_float(low) * pow2f(kTop - e) < kSmall);
                 (threadIdx.x < 32 ? aux.k_exp : aux.v_exp)[key] = e;
-                if (in && (bad || small)) atomicOr(&aux.odd[threadIdx.x >> 5], 1u << key);
+                if (in && threadIdx.x < 32 && (bad || small)) atomicOr(&aux.odd[0], 1u << key);
+                if (in && threadIdx.x >= 32 && bad) atomicOr(&aux.odd[1], 1u << key);
+                if (in && threadIdx.x >= 32 && small) atomicOr(&aux.odd[2], 1u << key);
             }
             float kf[NK][8], vf[NK][8];
             dequantize(k0, klo, khi, kf, vf);
@@ -1183,7 +1195,7 @@ struct SplitTile {
 #pragma unroll
                 for (int j = 0; j < 8; j++) {
                     const float sc = pow2f(kTop - aux.v_exp[v_piece_key(i, j)]);
-                    if (aux.odd[1] && v_is_odd(vf[r][j], sc)) vf[r][j] = 0.0f;
+                    if ((aux.odd[1] | aux.odd[2]) && (v_is_bad(vf[r][j]) || v_is_small(vf[r][j], sc))) vf[r][j] = 0.0f;
                     vf[r][j] *= sc;
                 }
                 split8(vf[r], 1.0f, hi, lo);
@@ -1214,9 +1226,16 @@ struct SplitTile {
                 const int e = class_of(top);
                 const float sc = pow2f(kTop - e);
                 if (top_bits(x) > top || __uint_as_float(low + 1u) * sc < kSmall) {
+                    bool bad = false, small = false;
 #pragma unroll
-                    for (int j = 0; j < 8; j++) x[j] = v_is_odd(x[j], sc) ? 0.0f : x[j];
-                    if (low != 0xffffffffu) atomicOr(&aux.odd[1], 1u << key);
+                    for (int j = 0; j < 8; j++) {
+                        const bool b = v_is_bad(x[j]), l = v_is_small(x[j], sc);
+                        bad = bad || b;
+                        small = small || l;
+                        x[j] = b || l ? 0.0f : x[j];
+                    }
+                    if (bad) atomicOr(&aux.odd[1], 1u << key);
+                    if (small) atomicOr(&aux.odd[2], 1u << key);
                 }
 #pragma unroll
                 for (int j = 0; j < 8; j++) x[j] *= sc;
@@ -1254,7 +1273,7 @@ struct SplitTile {
         if (threadIdx.x < 64) {
             const int key = threadIdx.x & 31;
             const int32_t exps = key_exps(aux.k_exp[key], aux.v_exp[key]);
-            const uint32_t odd_k = aux.odd[0], odd_v = aux.odd[1];
+            const uint32_t odd_k = aux.odd[0], bad_v = aux.odd[1], small_v = aux.odd[2];
             const int kp = k0 + key;
             const bool in = kp >= klo && kp <= khi;
             const uint32_t keys = (uint32_t)__ballot(in);
@@ -1262,8 +1281,8 @@ struct SplitTile {
             const bool same = !__ballot(in && exps != first);
             if (threadIdx.x < 32) aux.meta.exps[key] = exps;
             if (threadIdx.x == 0) {
-                aux.meta.head = TileHead{same ? first : kMixed, odd_k, odd_v};
-                aux.odd[0] = aux.odd[1] = 0;
+                aux.meta.head = TileHead{same ? first : kMixed, odd_k, bad_v, small_v};
+                aux.odd[0] = aux.odd[1] = aux.odd[2] = 0;
             }
         }
     }
@@ -1337,7 +1356,7 @@ __global__ __launch_bounds__(256) void stage_split_kernel(const PrefillParams p,
     const int b = blockIdx.x;
     const SeqTiles seq(p, b);
     __shared__ __attribute__((aligned(16))) SplitAux<D, Q8> aux;
-    if (threadIdx.x < 2) aux.odd[threadIdx.x] = 0;
+    if (threadIdx.x < 3) aux.odd[threadIdx.x] = 0;
     for (int item = blockIdx.y; item < seq.count * p.n_kv_heads; item += gridDim.y) {
         const int kvh = item / seq.count;
         const int t = item - kvh * seq.count;
@@ -1555,7 +1574,7 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill
         plain = exps != kMixed;
         for (int i = tid; i < n; i += 256) {
             const TileHead h = unit_meta[i].head;
-            plain = plain && h.exps == exps && !(h.odd_k | h.odd_v);
+            plain = plain && h.exps == exps && !(h.odd_k | h.bad_v | h.small_v);
         }
     }
 
@@ -1626,45 +1645,86 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill
     };
     // The f32 scores of a tile in place of the pieces' for odd keys and rows.
     const auto odd_scores = [&](floatx4 (&s)[2][NT], int k0, uint32_t keys) __attribute__((always_inline)) {
+        const PrefillParams *a = arguments();
+        const int64_t hb[2] = {head_page(a, k0), head_page(a, k0 + 16)};
+        const float *qp[NT];
 #pragma unroll
-        for (int mt = 0; mt < 2; mt++) {
-            floatx4 e[NT];
+        for (int nt = 0; nt < NT; nt++) {
+            const int lq = min(wq0 + nt * 16 + lrow, q_len - 1);  // (a row past the end has no result)
+            qp[nt] = a->q + ((int64_t)(row0 + lq) * a->n_heads + head) * D + lgrp * (D / 4);
+        }
+        floatx4 e[2][NT];
 #pragma unroll
-            for (int nt = 0; nt < NT; nt++) e[nt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-            const int kp = k0 + 16 * mt + lrow;
-            const bool have = kp >= ulo && kp <= uhi;
-            const PrefillParams *a = arguments();
-            const int64_t hb = head_page(a, k0 + 16 * mt);
-#pragma unroll 1
-            for (int step = 0; step < D / 4; step++) {
-                const int d = lgrp * (D / 4) + step;
-                const float kd = have ? k_element<D, Q8>(*a, hb, lrow, d) : 0.0f;
+        for (int mt = 0; mt < 2; mt++)
 #pragma unroll
-                for (int nt = 0; nt < NT; nt++) {
-                    const int lq = wq0 + nt * 16 + lrow;
-                    const bool ok = lq < q_len;
-                    const float x = a->q[((int64_t)(row0 + (ok ? lq : 0)) * a->n_heads + head) * D + d] * a->q_mul;
-                    e[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kd, ok ? x : 0.0f, e[nt], 0, 0, 0);
-                }
+            for (int nt = 0; nt < NT; nt++) e[mt][nt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 2
+        for (int d = 0; d < D / 4; d += 4) {  // lane group g multiplies the dims g * D/4 ..
+            floatx4 kd[2], qd[NT];
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) {
+                const int kp = k0 + 16 * mt + lrow;
+                kd[mt] = k_values4<D, Q8>(*a, hb[mt], lrow, lgrp * (D / 4) + d);
+                if (kp < ulo || kp > uhi) kd[mt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
             }
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) qd[nt] = *reinterpret_cast<const floatx4 *>(qp[nt] + d) * a->q_mul;
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+                    for (int nt = 0; nt < NT; nt++)
+                        e[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(kd[mt][j], qd[nt][j], e[mt][nt], 0, 0, 0);
+        }
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++)
 #pragma unroll
             for (int nt = 0; nt < NT; nt++)
 #pragma unroll
                 for (int r = 0; r < 4; r++)
-                    if (qodd[nt] || (keys >> (16 * mt + 4 * lgrp + r) & 1)) s[mt][nt][r] = e[nt][r];
+                    if (qodd[nt] || (keys >> (16 * mt + 4 * lgrp + r) & 1)) s[mt][nt][r] = e[mt][nt][r];
+    };
+    // The products of V's small values with the probabilities pv (element 4*mt + r
+    // of a lane: key 16*mt + 4*lgrp + r) on the f32 MFMA: its step (mt, r) takes
+    // those four keys.
+    const auto small_values = [&](const float (&pv)[NT][8], int k0, uint32_t keys, const TileMeta *meta) __attribute__((always_inline)) {
+        const PrefillParams *a = arguments();
+        const int64_t hb[2] = {head_page(a, k0), head_page(a, k0 + 16)};
+        float unit[NT];
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) unit[nt] = ldexpf(1.0f, kTop + kScaleP - rexp[nt]);
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int key = (j >> 2) * 16 + 4 * lgrp + (j & 3);
+            const bool has = keys >> key & 1;
+            const float scale = pow2f(kTop - v_exp_of(meta->exps[key]));
+            const LaneV<D, Q8> v(*a, hb[j >> 2], key & 15, lrow);
+            float x[DT];
+#pragma unroll
+            for (int t = 0; t < DT; t++) x[t] = v(t, 0);
+#pragma unroll
+            for (int t = 0; t < DT; t++) x[t] = has && v_is_small(x[t], scale) ? x[t] : 0.0f;
+#pragma unroll
+            for (int t = 0; t < DT; t++)
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++)
+                    o[t][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[t], pv[nt][j] * unit[nt], o[t][nt], 0, 0, 0);
         }
     };
-    // The products of V's odd values with the probabilities pv (element 4*mt + r
-    // of a lane: key 16*mt + 4*lgrp + r), for the queries that attend them.
-    const auto odd_values = [&](const float (&pv)[NT][8], int k0, uint32_t keys, const TileMeta *meta) __attribute__((always_inline)) {
+    // The products of V's infinities and NaN with the probabilities, for the
+    // queries that attend them.
+    const auto bad_values = [&](const float (&pv)[NT][8], int k0, uint32_t keys) __attribute__((always_inline)) {
         for (; keys; keys &= keys - 1) {
             const int key = __builtin_ctz(keys), reg = 4 * (key >> 4) + (key & 3);
             const int kp = k0 + key;
             const PrefillParams *a = arguments();
-            const int64_t hb = head_page(a, k0 + (key & 16));
-            
-            const float scale = pow2f(kTop - v_exp_of(meta->exps[key]));
-            const LaneV<D, Q8> v(*a, hb, key & 15, lgrp);
+            const LaneV<D, Q8> v(*a, head_page(a, k0 + (key & 16)), key & 15, 4 * lgrp);
+            float x[DT][4];
+#pragma unroll
+            for (int t = 0; t < DT; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) x[t][r] = v(t, r);
 #pragma unroll
             for (int nt = 0; nt < NT; nt++) {
                 float mine = pv[nt][0];
@@ -1675,11 +1735,8 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill
 #pragma unroll
                 for (int t = 0; t < DT; t++)
 #pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const float x = v(t, r);
-                        const float sum = fmaf(pk, ldexpf(x, kTop + kScaleP - rexp[nt]), o[t][nt][r]);
-                        o[t][nt][r] = attends && v_is_odd(x, scale) ? sum : o[t][nt][r];
-                    }
+                    for (int r = 0; r < 4; r++)
+                        o[t][nt][r] = attends && v_is_bad(x[t][r]) ? fmaf(pk, x[t][r], o[t][nt][r]) : o[t][nt][r];
             }
         }
     };
@@ -1842,8 +1899,10 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill
 #pragma unroll
         for (int nt = 0; nt < NT; nt++) add_cross(o[DT - 1][nt], cross[nt]);
         if constexpr (!same) {
-            const uint32_t odd_v = __builtin_amdgcn_readfirstlane(meta->head.odd_v);
-            if (odd_v) odd_values(pv, k0, odd_v, meta);
+            const uint32_t small_v = __builtin_amdgcn_readfirstlane(meta->head.small_v);
+            if (small_v) small_values(pv, k0, small_v, meta);
+            const uint32_t bad_v = __builtin_amdgcn_readfirstlane(meta->head.bad_v);
+            if (bad_v) bad_values(pv, k0, bad_v);
         }
     };
 
@@ -1876,7 +1935,7 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill
         constexpr bool AHEAD = D < 256;
         SplitTile<D, Q8> tile;
         tile.fetch(p, b, kvh, tfirst * KT, ulo, uhi);
-        if (tid < 2) aux.odd[tid] = 0;
+        if (tid < 3) aux.odd[tid] = 0;
         __syncthreads();
         const auto put = [&](int base) {
             uint8_t *to = lds + base;
@@ -1900,7 +1959,7 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill
             arrive(i);
             if (i == 0) exps = __builtin_amdgcn_readfirstlane(aux.meta.head.exps);
             here = exps == kMixed || __builtin_amdgcn_readfirstlane(aux.meta.head.exps) != exps ||
-                   __builtin_amdgcn_readfirstlane(aux.meta.head.odd_k | aux.meta.head.odd_v);
+                   __builtin_amdgcn_readfirstlane(aux.meta.head.odd_k | aux.meta.head.bad_v | aux.meta.head.small_v);
             if (here) break;
             attend(std::true_type{}, i, lds, nullptr);
         }

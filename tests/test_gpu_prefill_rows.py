@@ -112,7 +112,7 @@ def test_odd_values_reach_only_rows_that_attend_them(backend, d, H, Hkv, n):
 
 
 @pytest.mark.parametrize("n", [9, 20, 31, 45])
-@pytest.mark.parametrize("power", [-13, -16, -19, -25])
+@pytest.mark.parametrize("power", [-13, -16, -19, -25, -34])
 @pytest.mark.parametrize("d", [64, 128, 256])
 def test_small_dimensions_keep_their_precision(backend, d, n, power):
     """V dimensions far below the others, in tiles that are not full and beside full ones: each against 64 bits,
