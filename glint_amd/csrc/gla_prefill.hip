@@ -1693,7 +1693,8 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill
         const int64_t hb[2] = {head_page(a, k0), head_page(a, k0 + 16)};
         float unit[NT];
 #pragma unroll
-        for (int nt = 0; nt < NT; nt++) unit[nt] = ldexpf(1.0f, kTop + kScaleP - rexp[nt]);
+        for (int nt = 0; nt < NT; nt++)  // (a row that has attended no key has only zeros to multiply)
+            unit[nt] = rexp[nt] == kNoExp ? 0.0f : ldexpf(1.0f, kTop + kScaleP - rexp[nt]);
 #pragma unroll
         for (int j = 0; j < 8; j++) {
             const int key = (j >> 2) * 16 + 4 * lgrp + (j & 3);

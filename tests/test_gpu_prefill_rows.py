@@ -58,7 +58,7 @@ WHAT = ["q_inf", "q_spread", "k_inf", "k_spread", "k_large", "v_nan", "v_inf", "
 def test_rows_do_not_depend_on_their_neighbours(backend, dtype, what):
     """A prompt alone (one 16-query tile per wave), in a batch that fills the chip (two), and in pieces that are cut
     inside a 32-key tile and short enough to convert their own tiles: the same bits for every row."""
-    d, H, Hkv, n, at = 128, 8, 2, 700, 371
+    d, H, Hkv, n, at = 128, 8, 2, 900, 371
     lens = [n] + [n - 1] * 7
     k = synth.normal_rows(61, 8 * n, Hkv * d).reshape(8, 1, n, Hkv * d)
     v = synth.normal_rows(62, 8 * n, Hkv * d).reshape(8, 1, n, Hkv * d)
@@ -71,10 +71,30 @@ def test_rows_do_not_depend_on_their_neighbours(backend, dtype, what):
         both = run_prefill(backend, c.cache, q, start, [0] * 8, H, 0.09, None, window)[:n]
         alone = run_prefill(backend, c.cache, q[:n], [0, n], [0], H, 0.09, None, window, seq_slot=slot)
         assert _same(alone, both), (what, window, "alone")
-        for cuts in ([0, at - 3, at + 5, n], [0, 96, 160, 256, 340, at, at + 1, at + 40, 500, 596, n]):
+        for cuts in ([0, at - 3, at + 5, n], [0, 30, 62, 160, 256, 340, at, at + 1, at + 30, 500, 596, n]):
             got = [run_prefill(backend, c.cache, q[a:b], [0, b - a], [a], H, 0.09, None, window, seq_slot=slot)
                    for a, b in zip(cuts, cuts[1:])]
             assert _same(np.concatenate(got), both), (what, window, cuts)
+
+
+@pytest.mark.parametrize("what", ["q_inf", "k_inf", "v_nan", "v_inf"])
+@pytest.mark.parametrize("d,H,Hkv", [(64, 8, 2), (128, 8, 2), (256, 4, 2)])
+def test_bf16_nonfinite_data_is_batch_invariant(backend, d, H, Hkv, what):
+    """bf16 inputs: a prompt that starts inside a 32-key tile, with non-finite data beside its first rows, has the
+    same bits alone (one 16-query tile per wave) as in a batch that fills the chip (two)."""
+    n, off = 900 if d < 256 else 1700, 8
+    k = synth.normal_rows(65, 8 * (n + off), Hkv * d).reshape(8, 1, n + off, Hkv * d)
+    v = synth.normal_rows(66, 8 * (n + off), Hkv * d).reshape(8, 1, n + off, Hkv * d)
+    q = synth.normal(67, (8 * n, H, d))
+    for at in (40, 75, n - 20):
+        k2, v2, q2 = k.copy(), v.copy(), q.copy()
+        _plant(what, at, k2[0, 0], v2[0, 0], q2[:n])
+        c = Contig(backend, "f32", 8, 1, n + off, Hkv, d, k=k2, v=v2)
+        for window in (None, 50):
+            both = run_prefill(backend, c.cache, q2, np.arange(9) * n, [off] * 8, H, 0.09, None, window, precision="bf16")
+            alone = run_prefill(backend, c.cache, q2[:n], [0, n], [off], H, 0.09, None, window, precision="bf16",
+                                seq_slot=np.array([0], np.int32))
+            assert _same(alone, both[:n]), (what, at, window)
 
 
 @pytest.mark.parametrize("d,H,Hkv,n", [(64, 4, 2, 90), (128, 4, 2, 200), (256, 4, 2, 90)])
