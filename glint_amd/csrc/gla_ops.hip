@@ -582,14 +582,15 @@ __global__ __launch_bounds__(256) void gemm_q8_kernel(const uint8_t *quants, con
     }
     // scales of four row tiles by one copy: lanes 16t .. 16t+15 take tile t's 64 bytes
     const int stile = (wave * 4 + (lane >> 4)) % (2 * RT);
-    const uint32_t soff = (uint32_t)min(tile_wg + stile, n_tiles - 1) * (uint32_t)n_pairs * 64 + (lane & 15) * 4;
+    const uint8_t *sbase = reinterpret_cast<const uint8_t *>(scales) + (int64_t)tile_wg * n_pairs * 64;
+    const uint32_t soff = (uint32_t)min(stile, n_tiles - 1 - tile_wg) * (uint32_t)n_pairs * 64 + (lane & 15) * 4;
     const uint32_t sdst = (uint32_t)(wave * 4 % (2 * RT)) * 64;
     auto issue = [&](int p) {
         const uint32_t dst = ring + (uint32_t)(p % RING) * STAGE;
 #pragma unroll
         for (int c = 0; c < CPW; c++)
             lds_copy16(src[c] + (int64_t)p * step[c], lane * 16, dst + (wave * CPW + c) * 1024);
-        lds_copy4(reinterpret_cast<const uint8_t *>(scales) + (int64_t)p * 64, soff, dst + (WKB + XKB) * 1024 + sdst);
+        lds_copy4(sbase + (int64_t)p * 64, soff, dst + (WKB + XKB) * 1024 + sdst);
     };
 
     // this workgroup's slices, and their block pairs
