@@ -130,6 +130,42 @@ __device__ __forceinline__ bool arrive_last(int32_t *c, int n, int *lds_flag) {
     return *lds_flag != 0;
 }
 
+// Copies from global memory into LDS without registers: 16 (4) bytes per lane
+// from sbase + voff to m0 + 16 (4) * lane, m0 restored. Cached loads: what they
+// copy is read by many workgroups. The s_nop is the wait state an LDS-DMA load
+// needs after an SALU write of M0, which the compiler cannot insert into inline
+// assembly.
+__device__ __forceinline__ void lds_copy16(const uint8_t *sbase, uint32_t voff, uint32_t m0) {
+    uint32_t save;
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %3\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %1, %2\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(save)
+        : "v"(voff), "s"(sbase), "s"(m0)
+        : "memory");
+}
+__device__ __forceinline__ void lds_copy4(const uint8_t *sbase, uint32_t voff, uint32_t m0) {
+    uint32_t save;
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %3\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dword %1, %2\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(save)
+        : "v"(voff), "s"(sbase), "s"(m0)
+        : "memory");
+}
+// Wait until at most N of the wave's vector memory operations are in flight.
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+    static_assert(N >= 0 && N < 64, "vmcnt range");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
 __device__ __forceinline__ int64_t map_page(const PageMap &pm, int b, int lp) {
     int64_t id;
     if (pm.page_table) {
@@ -149,7 +185,7 @@ struct gla_ctx {
     int n_cu = 0;
     hipStream_t own_stream = nullptr;
     hipStream_t stream = nullptr;
-    // Device scratch (decode partials, bf16 tile images, matvec pieces), one
+    // Device scratch (decode partials, prefill tile images, matvec pieces), one
     // buffer per stream the context has launched work on: work queued on two
     // streams at once never shares a buffer.
     struct StreamScratch {

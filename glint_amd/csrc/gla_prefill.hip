@@ -597,42 +597,6 @@ constexpr int kRingTiles = D == 256 ? 4 : 3;
 template <int D>
 constexpr int kTileImage = 128 * D;
 
-// 16 bytes per lane from sbase + voff into LDS at m0 + 16*lane (m0 restored).
-// Default (cached) loads: each tile image is read by every query block of
-// its unit. The s_nop is the wait state an LDS-DMA load needs after an SALU
-// write of M0, which the compiler cannot insert into inline assembly.
-__device__ __forceinline__ void lds_copy16(const uint8_t *sbase, uint32_t voff, uint32_t m0) {
-    uint32_t save;
-    asm volatile(
-        "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %3\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %1, %2\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(save)
-        : "v"(voff), "s"(sbase), "s"(m0)
-        : "memory");
-}
-
-// 4 bytes per lane from sbase + voff into LDS at m0 + 4 * lane.
-__device__ __forceinline__ void lds_copy4(const uint8_t *sbase, uint32_t voff, uint32_t m0) {
-    uint32_t save;
-    asm volatile(
-        "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %3\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dword %1, %2\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(save)
-        : "v"(voff), "s"(sbase), "s"(m0)
-        : "memory");
-}
-
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-    static_assert(N >= 0 && N < 64, "vmcnt range");
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 // Waves per workgroup of the staged kernel (32 queries each): one per SIMD;
 // a CU holds several workgroups.
 template <int D>
