@@ -422,12 +422,12 @@ __device__ __forceinline__ void bf16_softmax(floatx4 (&sacc)[2][NT], float (&m)[
 
 // Row sums of the tile's bf16 probabilities, from one MFMA against an
 // all-ones operand: every element of a lane accumulates its query's sum.
-template <int NT, int FIRST = 0, int LAST = NT>
+template <int NT>
 __device__ __forceinline__ void bf16_row_sums(floatx4 (&lacc)[NT], const bf16x8 (&pb)[NT]) {
     const bf16x8 ones = bf16x8{(__bf16)1.0f, (__bf16)1.0f, (__bf16)1.0f, (__bf16)1.0f,
                                (__bf16)1.0f, (__bf16)1.0f, (__bf16)1.0f, (__bf16)1.0f};
 #pragma unroll
-    for (int nt = FIRST; nt < LAST; nt++) lacc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[nt], lacc[nt], 0, 0, 0);
+    for (int nt = 0; nt < NT; nt++) lacc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[nt], lacc[nt], 0, 0, 0);
 }
 
 template <int D, bool Q8, bool CAP>
@@ -741,26 +741,16 @@ __global__ __launch_bounds__(kBf16sWaves<D> * 64, kBf16sOccupancy<D>) void prefi
                         sacc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt], qb[nt][ks], sacc[mt][nt], 0, 0, 0);
             }
         };
-        // O^T += V^T . P^T, and the row sums, of the query tiles FIRST .. LAST-1
-        auto accumulate = [&](auto FIRST, auto LAST, const uint8_t *vimg, const bf16x8 (&pb)[NT]) __attribute__((always_inline)) {
-            bf16_row_sums<NT, FIRST, LAST>(lacc, pb);
+        // O^T += V^T . P^T, and the row sums
+        auto accumulate = [&](const uint8_t *vimg, const bf16x8 (&pb)[NT]) {
+            bf16_row_sums<NT>(lacc, pb);
 #pragma unroll
             for (int t = 0; t < DT; t++) {
                 const bf16x8 a = *reinterpret_cast<const bf16x8 *>(vimg + ((t * 4 + lgrp) * 16 + lrow) * 16);
 #pragma unroll
-                for (int nt = FIRST; nt < LAST; nt++)
+                for (int nt = 0; nt < NT; nt++)
                     o[t][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb[nt], o[t][nt], 0, 0, 0);
             }
-        };
-        const std::integral_constant<int, 0> zero;
-        const std::integral_constant<int, 1> one;
-        const std::integral_constant<int, NT> all;
-        // (a masked key's weight is 0, but 0 times an infinity or a NaN is not: a
-        // query tile takes only the tiles that some row of it attends, as it does
-        // in a wave of its own)
-        const auto attends = [&](int nt, int k0) __attribute__((always_inline)) {
-            return k0 <= min(khi, pos0 + wq0 + 16 * nt + 15) &&
-                   k0 + KT - 1 >= max(klo, window_lo(pos0 + wq0 + 16 * nt, p.sliding_window));
         };
         // The leading tiles inside the causal and window bounds of every query
         // of the workgroup, when its waves share one query block (one q-head
@@ -780,7 +770,7 @@ __global__ __launch_bounds__(kBf16sWaves<D> * 64, kBf16sOccupancy<D>) void prefi
             scores(kimg, sacc);
             bf16x8 pb[NT];
             bf16_softmax_interior<NT, DT, CAP>(sacc, m, lacc, o, pb, p.softcap);
-            accumulate(zero, all, kimg + 64 * D, pb);
+            accumulate(kimg + 64 * D, pb);
         }
         for (; i < n; i++) {
             arrive(i);
@@ -796,8 +786,7 @@ __global__ __launch_bounds__(kBf16sWaves<D> * 64, kBf16sOccupancy<D>) void prefi
             bf16x8 pb[NT];
             bf16_softmax<NT, DT, CAP>(sacc, m, lacc, o, pb, p.softcap, interior, k0 + 4 * lgrp, qpos, qlo, klo,
                                       khi);
-            if (NT == 1 || attends(0, k0)) accumulate(zero, one, kimg + 64 * D, pb);
-            if (NT == 2 && attends(1, k0)) accumulate(one, all, kimg + 64 * D, pb);
+            accumulate(kimg + 64 * D, pb);
         }
     }
 
