@@ -644,9 +644,12 @@ __global__ __launch_bounds__(kBf16sWaves<D> * 64, kBf16sOccupancy<D>) void prefi
     const int head = kvh * p.group + hgrp * p.hpw + (wave % p.hpw);
     const int wq0 = qb0 + (wave / p.hpw) * QW;
 
-    const int q_last = min(q_len, qb0 + qwg) - 1;
+    // The keys are those of whole blocks of 32 rows, also where a wave takes 16:
+    // 0 times an infinity or a NaN of V is not 0, so which masked keys a row's tiles
+    // hold must not depend on NT
+    const int q_last = min(q_len, (qb0 + qwg + 31) & ~31) - 1;
     const int khi = min(pos0 + q_last, p.pm.pos_limit - 1);
-    const int klo = window_lo(pos0 + qb0, p.sliding_window);
+    const int klo = window_lo(pos0 + (qb0 & ~31), p.sliding_window);
 
     bf16x8 qb[NT][KS];
 #pragma unroll
@@ -681,9 +684,9 @@ __global__ __launch_bounds__(kBf16sWaves<D> * 64, kBf16sOccupancy<D>) void prefi
         qpos[nt] = lq < q_len ? pos0 + lq : -1;
         qlo[nt] = window_lo(pos0 + lq, p.sliding_window);
     }
-    // keys this wave's queries attend: [wlo, whi]
-    const int whi = min(khi, pos0 + wq0 + QW - 1);
-    const int wlo = max(klo, window_lo(pos0 + wq0, p.sliding_window));
+    // keys that the wave's block of 32 rows attends: [wlo, whi]
+    const int whi = min(khi, pos0 + (wq0 | 31));
+    const int wlo = max(klo, window_lo(pos0 + (wq0 & ~31), p.sliding_window));
 
     if (khi >= klo) {
         const int tfirst = klo / KT;
