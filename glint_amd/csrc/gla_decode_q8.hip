@@ -798,8 +798,8 @@ __device__ __forceinline__ void wave_chunk(const Q8Params &p, const Range &r, in
 // Pages per workgroup of a window of n pages: `full`, but a window of two
 // workgroups is cut in half, so that neither walks longer than it has to. Four
 // sequences of 200-2,000 positions at 32/8 heads, d = 128 (125 pages: 112 + 13
-// before): 25.6 -> 20.6 us per call, 16 of 1,900-2,500 66 -> 56, 64 of
-// 128-8,192 96.2 -> 95.2. Windows of three workgroups and more keep full ones:
+// before): 25.6 -> 20.6 us per call, 16 of 1,900-2,500 66 -> 56; 64 of
+// 128-8,192 are within the runs' difference. Windows of three workgroups and more keep full ones:
 // cut evenly, the last batch takes 96.1, and so does head_dim 256 (32 Gemma-2 sequences of 2,048-8,192, a
 // window and a global layer: 199.6 -> 214.6). A rule on the window alone, as
 // batch invariance needs.

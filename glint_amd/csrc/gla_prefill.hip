@@ -834,7 +834,7 @@ __global__ __launch_bounds__(kBf16sWaves<D> * 64, kBf16sOccupancy<D>) void prefi
 // eight times, so the error against 64 bits is smaller: 4 prompts of 2,048 at
 // 32/8 heads, d = 128, 2.0e-7 relative (f32 MFMAs: 4.4e-7). Three f16 MFMAs do
 // the work of a 16x16x32 tile in 48 cycles, the f32 ones in 256: the same four
-// prompts take 394 us, of them 23 the staging (f32 MFMAs: 1,083 us). What bounds
+// prompts take 400 us, of them 23 the staging (f32 MFMAs: 1,083 us). What bounds
 // it is the chain S -> softmax -> O at two waves per SIMD: matrix and vector
 // cycles add up.
 //
@@ -847,17 +847,17 @@ __global__ __launch_bounds__(kBf16sWaves<D> * 64, kBf16sOccupancy<D>) void prefi
 // exponent and R the row's: the largest E it has attended, moved (with O) when
 // one passes it by more than 2^2. So the products' operand is largest where the
 // contribution p * V is, and it is the small contributions that reach the end of
-// f16's range. Where all keys that a workgroup attends share their exponents and
-// nothing is odd, as with most data, its loop over the tiles holds the scales as
-// constants (`plain`); otherwise it takes them key by key. Both give the same bits.
+// f16's range. Tiles whose keys share the exponents of the first that has the same
+// for all and hold nothing odd, as with most data, are taken by a loop that holds
+// the scales as constants; the others key by key. Both give the same bits.
 //
 // What the pieces cannot hold is named per key ("odd"): infinities and NaN, K
 // with a run of 8 dims below 2^-20 of its largest value, V's values below kSmall
 // (scaled). The scores of an odd key, or of a query row that is odd in the same
 // way, come from the f32 MFMA. Odd V values are zero in the image; the small
 // ones' products are added by the f32 MFMA, the others' for the rows that attend
-// them. us per call of 4 x 2,048 rows, 32/8 heads, d = 128: 394 where nothing
-// differs, 480 where the keys' exponents differ, 510 with a NaN in V, 1,400 with every
+// them. us per call of 4 x 2,048 rows, 32/8 heads, d = 128: 400 where nothing
+// differs, 410 with a NaN or a small value in V, 490 where every tile's keys differ, 1,400 with every
 // 16th dim of V at 2^-34 of the others, 2,200 with eight dims of every key at 2^-30
 // (f32 MFMAs for everything: 1,080).
 typedef _Float16 half8p __attribute__((ext_vector_type(8)));
@@ -1533,16 +1533,13 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill
     };
 
     if (STAGED && n > 0) issue(0);
-    // whether the tiles' keys share their exponents and none is odd
-    bool plain = true;
+    // the exponents of the first tile whose keys share them (a prompt's first keys
+    // often differ from the rest)
     int32_t exps = kMixed;
-    if (STAGED && n > 0) {
-        exps = __builtin_amdgcn_readfirstlane(unit_meta[0].head.exps);
-        plain = exps != kMixed;
-        for (int i = tid; i < n; i += 256) {
-            const TileHead h = unit_meta[i].head;
-            plain = plain && h.exps == exps && !(h.odd_k | h.bad_v | h.small_v);
-        }
+    for (int i = 0; STAGED && i < n && exps == kMixed; i += 64) {
+        const int32_t mine = unit_meta[min(i + lane, n - 1)].head.exps;
+        const uint64_t found = __ballot(mine != kMixed);
+        if (found) exps = __builtin_amdgcn_readlane(mine, __builtin_ctzll(found));
     }
 
     // Q^T operand: pieces of Q[query nt*16 + lrow][d = ks*32 + lgrp*8 + 0..7]
@@ -1579,11 +1576,12 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill
         qodd[nt] = umax_rows4(bad);
         any_odd = any_odd || __ballot(qodd[nt]);
     }
-    plain = !__syncthreads_or(any_odd || !plain);
+    const bool plain = !__syncthreads_or(any_odd) && (!STAGED || exps != kMixed);
 
     floatx4 o[DT][NT];
     float m[NT], lpart[NT];
     int rexp[NT];  // R: O is in units of 2^(rexp - kTop - kScaleP)
+    float weight[NT];  // 2^(E - R + kScaleP) of `exps`
     int qpos[NT], qlo[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; nt++) {
@@ -1591,6 +1589,7 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill
         for (int t = 0; t < DT; t++) o[t][nt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
         lpart[nt] = 0.0f;
         rexp[nt] = kNoExp;
+        weight[nt] = (float)(1 << kScaleP);
         m[nt] = kMLowest;  // finite: the first attended key is an ordinary move of the reference
         const int lq = wq0 + nt * 16 + lrow;
         qpos[nt] = lq < q_len ? pos0 + lq : -1;
@@ -1813,7 +1812,7 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill
             float x[8];
             if constexpr (same) {
 #pragma unroll
-                for (int j = 0; j < 8; j++) x[j] = pv[nt][j] * (float)(1 << kScaleP);
+                for (int j = 0; j < 8; j++) x[j] = pv[nt][j] * weight[nt];
             } else {
                 const int lo = max(qlo[nt], klo), hi = min(qpos[nt], khi);
                 int top = kNoExp;  // of the keys that the row attends
@@ -1882,20 +1881,49 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill
             __syncthreads();
             if (i + 1 < n) issue(i + 1);
         };
-        if (plain) {
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++) rexp[nt] = v_exp_of(exps);
-            for (int i = 0; i < n; i++) {
-                arrive(i);
-                attend(std::true_type{}, i, lds + (i & 1) * IMG, nullptr);
+        // the first tile from `i` on whose keys have other exponents than `exps` or
+        // hold something odd
+        const auto next_special = [&](int i) __attribute__((always_inline)) {
+            if (!plain) return i;
+            for (; i < n; i += 64) {
+                const TileHead h = unit_meta[min(i + lane, n - 1)].head;
+                const uint64_t found = __ballot(h.exps != exps || (h.odd_k | h.bad_v | h.small_v));
+                if (found) return min(n, i + __builtin_ctzll(found));
             }
-        } else {
-            const TileMeta *metas = reinterpret_cast<const TileMeta *>(lds + METAS);
-            if (n > 0) issue_meta(0);
-            for (int i = 0; i < n; i++) {
+            return n;
+        };
+        const TileMeta *metas = reinterpret_cast<const TileMeta *>(lds + METAS);
+        for (int i = 0; i < n;) {
+            const int stop = next_special(i);
+            if (i < stop) {
+                // R as the first of these tiles would have it, for the rows that
+                // attend it; a row that has attended nothing may take it early
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++) {
+                    const int e = v_exp_of(exps);
+                    const bool up = e > rexp[nt] + kLazyExp &&
+                                    (rexp[nt] == kNoExp || qpos[nt] >= (tfirst + i) * KT);
+                    if (__ballot(up && rexp[nt] != kNoExp)) {
+                        const float f = up && rexp[nt] != kNoExp ? ldexpf(1.0f, rexp[nt] - e) : 1.0f;
+#pragma unroll
+                        for (int t = 0; t < DT; t++) o[t][nt] *= f;
+                    }
+                    rexp[nt] = up ? e : rexp[nt];
+                    weight[nt] = ldexpf(1.0f, min(e - rexp[nt], kLazyExp) + kScaleP);
+                }
+                for (; i < stop; i++) {
+                    arrive(i);
+                    attend(std::true_type{}, i, lds + (i & 1) * IMG, nullptr);
+                }
+            }
+            if (i < n) {
+                // (a row that has attended a key has moved its maximum)
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++) rexp[nt] = m[nt] != kMLowest ? rexp[nt] : kNoExp;
+                issue_meta(i);
                 arrive(i);
-                if (i + 1 < n) issue_meta(i + 1);
                 attend(std::false_type{}, i, lds + (i & 1) * IMG, metas + (i & 1));
+                i++;
             }
         }
     } else if (n > 0) {

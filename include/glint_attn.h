@@ -57,7 +57,11 @@ typedef enum gla_kv_dtype { GLA_KV_F32 = 0, GLA_KV_Q8_0 = 1 } gla_kv_dtype;
 
 /* Arithmetic of the prefill matrix products. */
 typedef enum gla_precision {
-    GLA_PREC_F32 = 0, /* fp32 inputs, fp32-accumulate MFMA */
+    GLA_PREC_F32 = 0, /* fp32: every operand as two f16 pieces (22 bits at any
+                         magnitude), three f16 MFMAs a product, fp32
+                         accumulation; closer to 64 bits than fp32 MFMAs. A
+                         query row's bits follow from the row and the keys it
+                         attends alone. */
     GLA_PREC_BF16 = 1 /* bf16-rounded Q/K/P/V inputs, fp32-accumulate MFMA */
 } gla_precision;
 
@@ -342,8 +346,9 @@ int gla_q8w_cols(const gla_q8w *w);
 /* y[v][r] = sum_c W[r][c] * x[v][c] for n_vec vectors: QuantizedTensor::matvec
  * and matvec_batch over Q8_0 (src/tensor/quantized.rs:247-346, :587-610; the
  * wgpu matvec_q8_0 shader's job). x device [n_vec][cols], y device
- * [n_vec][rows], f32. Asynchronous; the weights are read once per 64
- * vectors. n_vec above 262,128 is refused (GLA_ERR_INVALID): split the call. */
+ * [n_vec][rows], f32. Asynchronous; up to 64 vectors read the weights
+ * once, more share them in tiles through LDS. n_vec above 262,128 is refused
+ * (GLA_ERR_INVALID): split the call. */
 int gla_matvec_q8_0(gla_ctx *ctx, const gla_q8w *w, const float *x, int n_vec, float *y);
 
 #ifdef __cplusplus

@@ -43,6 +43,12 @@ def _plant(what, at, k, v, q):
     elif what == "v_spread":  # one run small beside the rest of a tile: 2^-14, then 2^-30
         v[at, ::16] *= np.float32(2.0**-14)
         v[at + 1, 1::16] *= np.float32(2.0**-30)
+    elif what == "sink":  # the first key's K large and its V small, the next ones' V smaller yet
+        k[0] *= np.float32(100.0)
+        v[0] *= np.float32(2.0**-9)
+        v[1:40] *= np.float32(2.0**-17)
+    elif what == "v_tiny":  # rows that attend only these have outputs of 2^-100
+        v[:64] *= np.float32(2.0**-100)
     elif what == "v_zero":
         v[at:at + 40] = 0.0
     elif what == "v_max":  # bf16 would round it to infinity; the output is finite
@@ -50,7 +56,7 @@ def _plant(what, at, k, v, q):
 
 
 WHAT = ["q_inf", "q_spread", "k_inf", "k_spread", "k_large", "v_nan", "v_inf", "v_large", "v_small", "v_spread",
-        "v_zero", "v_max"]
+        "sink", "v_tiny", "v_zero", "v_max"]
 
 
 @pytest.mark.parametrize("dtype", ["f32", "q8"])
