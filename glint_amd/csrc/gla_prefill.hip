@@ -862,6 +862,8 @@ __global__ __launch_bounds__(kBf16sWaves<D> * 64, kBf16sOccupancy<D>) void prefi
 // (f32 MFMAs for everything: 1,080).
 typedef _Float16 half8p __attribute__((ext_vector_type(8)));
 
+// instruction groups for the scheduler: MFMAs, LDS reads
+constexpr int kSchedMfma = 0x8, kSchedLds = 0x100;
 constexpr float kMLowest = -3.402823466e38f;  // a row's maximum before its first key
 constexpr float kLazyF32 = 4.0f;  // the lazy maximum's margin: p = 2^(s - m) stays below 2^4, whatever m's ulp
 constexpr int kLazyExp = 2;       // R's: p * 2^(E - R) stays below 2^6
@@ -1750,6 +1752,14 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill
                     x[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[mt], qh[nt][ks], x[mt][nt], 0, 0, 0);
         }
 
+        // operands of the next d step in flight while one is multiplied
+        __builtin_amdgcn_sched_group_barrier(kSchedLds, 8, 0);
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            __builtin_amdgcn_sched_group_barrier(kSchedMfma, 6 * NT, 0);
+            if (ks + 2 < KS) __builtin_amdgcn_sched_group_barrier(kSchedLds, 4, 0);
+        }
+
         // softmax: as the bf16 kernels' (a lazy maximum), in f32; c undoes the scales
         const bool interior = k0 >= klo && k0 + KT - 1 <= min(khi, pos0 + wq0) &&
                               (p.sliding_window <= 0 || k0 >= window_lo(pos0 + wq0 + QW - 1, p.sliding_window));
@@ -1865,6 +1875,12 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill
         }
 #pragma unroll
         for (int nt = 0; nt < NT; nt++) add_cross(o[DT - 1][nt], cross[nt]);
+        __builtin_amdgcn_sched_group_barrier(kSchedLds, 4, 1);
+#pragma unroll
+        for (int t = 0; t < DT; t++) {
+            __builtin_amdgcn_sched_group_barrier(kSchedMfma, 3 * NT, 1);
+            if (t + 2 < DT) __builtin_amdgcn_sched_group_barrier(kSchedLds, 2, 1);
+        }
         if constexpr (!same) {
             const uint32_t small_v = __builtin_amdgcn_readfirstlane(meta->head.small_v);
             if (small_v) small_values(pv, k0, small_v, meta);
@@ -1893,8 +1909,17 @@ __global__ __launch_bounds__(256, (kSplitOccupancy<D, STAGED, NT>)) void prefill
             return n;
         };
         const TileMeta *metas = reinterpret_cast<const TileMeta *>(lds + METAS);
-        for (int i = 0; i < n;) {
-            const int stop = next_special(i);
+        int stop = n > 0 ? next_special(0) : 0;
+        if (stop == n) {  // (the usual case in a loop of its own, whose registers nothing else shares)
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) rexp[nt] = v_exp_of(exps);
+            for (int i = 0; i < n; i++) {
+                arrive(i);
+                attend(std::true_type{}, i, lds + (i & 1) * IMG, nullptr);
+            }
+            stop = -1;
+        }
+        for (int i = 0; stop >= 0 && i < n; stop = i < n ? next_special(i) : 0) {
             if (i < stop) {
                 // R as the first of these tiles would have it, for the rows that
                 // attend it; a row that has attended nothing may take it early
@@ -2063,11 +2088,13 @@ constexpr int kRounds = 4;
 // Query rows of a call's longest sequence, and tiles of its storage, up to which
 // workgroups convert their own tiles: the second launch costs such a call more than
 // the repeated conversion. One sequence, us per call, unstaged / staged: from
-// position 0, d = 128 20 rows 9.2 / 11.5, 90 rows 15.5 / 14.5; d = 64 20 rows 7.1 /
-// 9.4; d = 256 20 rows 13.4 / 15.2; after 300 cached positions 20 rows 36 / 22,
-// after 4,000 387 / 151.
-constexpr int kUnstagedRows = 32;
-constexpr int kUnstagedTiles = 4;
+// position 0, d = 128 20 rows 9.2 / 11.5, 60 rows 12.4 / 13.6, 90 rows 15.5 / 14.5;
+// d = 64 20 rows 7.1 / 9.4, 50 rows 9.3 / 10.8; d = 256 20 rows 13.4 / 15.2, 40 rows
+// 18.8 / 17.3; after 300 cached positions, d = 128, 20 rows 36 / 22, after 4,000
+// 387 / 151.
+template <int D>
+constexpr int kUnstagedRows = D == 256 ? 32 : 64;
+constexpr int kUnstagedTiles = 3;
 
 template <int D, bool Q8, bool CAP, bool STAGED, int NT>
 int launch_split_as(gla_ctx *ctx, PrefillParams prm, int n_units, const Images &im) {
@@ -2092,7 +2119,7 @@ int launch_split(gla_ctx *ctx, const PrefillParams &prm, int n_seqs, int n_hgrp,
     if (prm.sliding_window > 0)
         n_tiles = (int)std::min<int64_t>(n_tiles, ((int64_t)prm.max_q_len + prm.sliding_window - 2) / KT + 2);
     constexpr size_t per = kSplitImage<D> + sizeof(TileMeta);
-    const bool few = prm.max_q_len <= kUnstagedRows && n_tiles <= kUnstagedTiles;
+    const bool few = prm.max_q_len <= kUnstagedRows<D> && n_tiles <= kUnstagedTiles;
     Images im{};
     im.rounds = 1;
     bool all_placed = true;

@@ -83,6 +83,27 @@ def test_rows_do_not_depend_on_their_neighbours(backend, dtype, what):
             assert _same(np.concatenate(got), both), (what, window, cuts)
 
 
+@pytest.mark.parametrize("dtype", ["f32", "q8"])
+@pytest.mark.parametrize("d,H,Hkv", [(64, 9, 3), (128, 8, 2), (256, 4, 2)])
+def test_workgroups_that_convert_give_the_staged_bits(backend, d, H, Hkv, dtype):
+    """A storage of three tiles: a prompt of all its rows is staged, one in pieces of up to 32 rows converts its
+    tiles in the workgroups."""
+    n = 96
+    for at in (0, 37, 60):
+        for what in WHAT:
+            k = synth.normal_rows(76, n, Hkv * d).reshape(1, 1, n, Hkv * d)
+            v = synth.normal_rows(77, n, Hkv * d).reshape(1, 1, n, Hkv * d)
+            q = synth.normal(78, (n, H, d))
+            _plant(what, at, k[0, 0], v[0, 0], q)
+            c = Contig(backend, dtype, 1, 1, n, Hkv, d, k=k, v=v)
+            for cap, window in ((None, None), (20.0, 37)):
+                one = run_prefill(backend, c.cache, q, [0, n], [0], H, 0.1, cap, window)
+                cuts = [0, 1, 30, 40, 41, 72, n]
+                got = [run_prefill(backend, c.cache, q[a:b], [0, b - a], [a], H, 0.1, cap, window)
+                       for a, b in zip(cuts, cuts[1:])]
+                assert _same(np.concatenate(got), one), (what, at, cap, window)
+
+
 @pytest.mark.parametrize("what", ["q_inf", "k_inf", "v_nan", "v_inf"])
 @pytest.mark.parametrize("d,H,Hkv", [(64, 8, 2), (128, 8, 2), (256, 4, 2)])
 def test_bf16_nonfinite_data_is_batch_invariant(backend, d, H, Hkv, what):
