@@ -857,7 +857,7 @@ __global__ __launch_bounds__(kBf16sWaves<D> * 64, kBf16sOccupancy<D>) void prefi
 // way, come from the f32 MFMA. Odd V values are zero in the image; the small
 // ones' products are added by the f32 MFMA, the others' for the rows that attend
 // them. us per call of 4 x 2,048 rows, 32/8 heads, d = 128: 400 where nothing
-// differs, 410 with a NaN or a small value in V, 490 where every tile's keys differ, 1,400 with every
+// differs, 410 with a NaN in V, 430 with a small value, 500 where every tile's keys differ, 1,400 with every
 // 16th dim of V at 2^-34 of the others, 2,200 with eight dims of every key at 2^-30
 // (f32 MFMAs for everything: 1,080).
 typedef _Float16 half8p __attribute__((ext_vector_type(8)));
